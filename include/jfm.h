@@ -585,6 +585,7 @@ int32_t jfm_mutual_combine(void* stream, int32_t dtype, int32_t n, const void* m
  *   op 2 l2l (in: local,     delta = parent - child)
  *   op 3 p2m (in[0]: mass,   delta = particle - centre)
  *   op 4 l2p (in: local,     delta = centre - point; out = phi, dphi/ddelta[3])
+ *   op 5 m2l by the rotation cascade (the matrix-core engine's form), else as op 1
  * in/out hold (p+1)^2 doubles; dtype selects the arithmetic precision. */
 int32_t jfm_host_operator(int32_t op, int32_t p, int32_t dtype, const double* in, const double* delta, double* out);
 

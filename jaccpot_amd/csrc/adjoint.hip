@@ -29,6 +29,7 @@
 #include "device_math.hpp"
 #include "launch.hpp"
 #include "rows.hpp"
+#include "translate.hpp"
 
 // Orders with adjoint kernels (every order of the forward path; the centre
 // pass translates at order p + 1, for which the B_U tables reach degree 9).
@@ -380,11 +381,7 @@ __device__ __forceinline__ void m2l_bilinear_grad(const T* A, const T* B, T dx, 
   constexpr int C = ncoef(P), C1 = ncoef(P + 1);
   T v[C1], w[C1];
   for (int j = 0; j < C1; ++j) v[j] = j < C ? B[j] : T(0);
-  Align<T, P + 1> a;
-  a.init(dx, dy, dz);
-  rotate_all<T, P + 1, Rot::ToZMultipole>(v, a);
-  zm2l<T, P + 1>(v, w, a.r);
-  rotate_all<T, P + 1, Rot::FromZLocal>(w, a);
+  m2l<T, P + 1, P>(v, w, dx, dy, dz);
   T Gx[C], Gy[C], Gz[C];
   grad_coeffs<T, P + 1>(w, Gx, Gy, Gz);
   T sx = T(0), sy = T(0), sz = T(0);

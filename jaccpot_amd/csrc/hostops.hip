@@ -7,6 +7,7 @@
 
 #include "device_math.hpp"
 #include "launch.hpp"
+#include "translate.hpp"
 
 namespace jfm {
 namespace {
@@ -39,24 +40,20 @@ void host_op(int32_t op, const double* in, const double* delta, double* out) {
     out[3] = gz;
     return;
   }
-  Align<T, P> a;
-  a.init(dx, dy, dz);
   if (op == 0) {  // m2m, delta = source - destination
-    rotate_all<T, P, Rot::ToZMultipole>(v, a);
-    zshift_m2m<T, P>(v, a.r);
-    rotate_all<T, P, Rot::FromZMultipole>(v, a);
-    for (int j = 0; j < C; ++j) out[j] = v[j];
+    m2m<T, P>(v, w, dx, dy, dz);
   } else if (op == 1) {  // m2l, delta = target - source
+    m2l<T, P>(v, w, dx, dy, dz);
+  } else if (op == 2) {  // l2l, delta = parent - child
+    l2l<T, P>(v, w, dx, dy, dz);
+  } else {  // m2l by the rotation cascade (the matrix-core engine's form)
+    Align<T, P> a;
+    a.init(dx, dy, dz);
     rotate_all<T, P, Rot::ToZMultipole>(v, a);
     zm2l<T, P>(v, w, a.r);
     rotate_all<T, P, Rot::FromZLocal>(w, a);
-    for (int j = 0; j < C; ++j) out[j] = w[j];
-  } else {  // l2l, delta = parent - child
-    rotate_all<T, P, Rot::ToZLocal>(v, a);
-    zshift_l2l<T, P>(v, a.r);
-    rotate_all<T, P, Rot::FromZLocal>(v, a);
-    for (int j = 0; j < C; ++j) out[j] = v[j];
   }
+  for (int j = 0; j < C; ++j) out[j] = static_cast<double>(w[j]);
 }
 
 }  // namespace
@@ -64,7 +61,7 @@ void host_op(int32_t op, const double* in, const double* delta, double* out) {
 
 extern "C" int32_t jfm_host_operator(int32_t op, int32_t p, int32_t dtype, const double* in, const double* delta,
                                      double* out) {
-  if (op < 0 || op > 4) return jfm::fail(JFM_ERR_ARG, "jfm_host_operator: op must be 0..4");
+  if (op < 0 || op > 5) return jfm::fail(JFM_ERR_ARG, "jfm_host_operator: op must be 0..5");
   if (!in || !delta || !out) return jfm::fail(JFM_ERR_ARG, "jfm_host_operator: NULL buffer");
   JFM_FOR_DTYPE(dtype, JFM_FOR_ORDER(p, { jfm::host_op<T, P>(op, in, delta, out); }));
   return JFM_OK;

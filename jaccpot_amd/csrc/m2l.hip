@@ -18,6 +18,7 @@
 #include "device_math.hpp"
 #include "launch.hpp"
 #include "rows.hpp"
+#include "translate.hpp"
 #include "xcd.hpp"
 
 namespace jfm {
@@ -157,67 +158,27 @@ __device__ __forceinline__ void rotate_all_mf(float* v, const Align<float, P>& a
   }
 }
 
-// One pair's M2L contribution w = D_from^L Z(r) D_to^M v at order G (v is
-// overwritten); MF: B_U on the matrix cores (float32 only), else the VALU.
+// One pair's M2L contribution w at order G (v is overwritten); MF: the rotation
+// cascade with B_U on the matrix cores (float32 only), else translate.hpp's form.
 template <typename T, int G, bool MF>
 __device__ __forceinline__ void m2l_pair(T* v, T* w, T dx, T dy, T dz, const BuRegs& bu) {
-  Align<T, G> a;
-  a.init(dx, dy, dz);
   if constexpr (MF) {
     static_assert(sizeof(T) == 4, "matrix-core B_U is float32 only");
+    Align<T, G> a;
+    a.init(dx, dy, dz);
     rotate_all_mf<G, Rot::ToZMultipole>(v, a, bu);
     zm2l<T, G>(v, w, a.r);
     rotate_all_mf<G, Rot::FromZLocal>(w, a, bu);
   } else {
-    rotate_all<T, G, Rot::ToZMultipole>(v, a);
-    zm2l<T, G>(v, w, a.r);
-    rotate_all<T, G, Rot::FromZLocal>(w, a);
+    m2l<T, G>(v, w, dx, dy, dz);
   }
 }
 
-// G <= P is the pair's expansion order (gear): the source multipole is read
-// to degree G, translated at order G and added into degrees <= G of the
-// target local.  ACC adds into the existing rows instead of overwriting them
-// (used when a target's pairs are split across several gears).
-template <typename T, int P, int G, bool ACC, bool MF>
-__global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ targets,
-                                                    const int32_t* __restrict__ far_off,
-                                                    const int32_t* __restrict__ far_src, const T* __restrict__ mult,
-                                                    const T* __restrict__ centers4, T* __restrict__ locals,
-                                                    int32_t cs) {
-  constexpr int C = ncoef(G);
+// Sum of the lanes' coefficients acc[C] added to (ACC) or stored in `row`,
+// through LDS, CH coefficients at a time, lanes in order.
+template <typename T, int C, bool ACC>
+__device__ __forceinline__ void reduce_lanes(const T* acc, T (*red)[row_for(C, sizeof(T))], T* row, int lane) {
   constexpr int CH = chunk_for(C, sizeof(T));
-  __shared__ T red[kWave][row_for(C, sizeof(T))];
-  const int tgt = targets[xcd_contiguous(blockIdx.x, gridDim.x)];
-  const int lane = threadIdx.x;
-  BuRegs bu;
-  if constexpr (MF) bu.load(lane);
-  const int b = far_off[tgt], e = far_off[tgt + 1];
-  const V4<T> ct = load4(centers4, tgt);
-  T acc[C];
-#pragma unroll
-  for (int j = 0; j < C; ++j) acc[j] = T(0);
-  // MF: the matrix instructions need every lane of the wave, so the loop runs
-  // to the wave's last round; lanes past the list repeat the target's first
-  // pair and drop the result
-  const int rounds = (e - b + kWave - 1) / kWave;
-  for (int q = 0; q < rounds; ++q) {
-    const int k = b + q * kWave + lane;
-    if (!MF && k >= e) break;
-    const bool live = k < e;
-    const int src = far_src[live ? k : b];
-    const V4<T> cs4 = load4(centers4, src);
-    T v[C];
-    load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
-    T w[C];
-    m2l_pair<T, G, MF>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
-    if (live) {
-#pragma unroll
-      for (int j = 0; j < C; ++j) acc[j] += w[j];
-    }
-  }
-  // lane partial sums reduced through LDS, CH coefficients at a time
-  T* row = locals + static_cast<int64_t>(tgt) * cs;
 #pragma unroll
   for (int c0 = 0; c0 < C; c0 += CH) {
     __syncthreads();
@@ -234,6 +195,73 @@ __global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ 
         row[c0 + lane] = s;
     }
   }
+}
+
+// G <= P is the pair's expansion order (gear): the source multipole is read
+// to degree G, translated at order G and added into degrees <= G of the
+// target local.  ACC adds into the existing rows instead of overwriting them
+// (used when a target's pairs are split across several gears).
+template <typename T, int P, int G, bool ACC, bool MF>
+__global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ targets,
+                                                    const int32_t* __restrict__ far_off,
+                                                    const int32_t* __restrict__ far_src, const T* __restrict__ mult,
+                                                    const T* __restrict__ centers4, T* __restrict__ locals,
+                                                    int32_t cs) {
+  constexpr int C = ncoef(G);
+  __shared__ T red[kWave][row_for(C, sizeof(T))];
+  const int tgt = targets[xcd_contiguous(blockIdx.x, gridDim.x)];
+  const int lane = threadIdx.x;
+  BuRegs bu;
+  if constexpr (MF) bu.load(lane);
+  const int b = far_off[tgt], e = far_off[tgt + 1];
+  const V4<T> ct = load4(centers4, tgt);
+  T* row = locals + static_cast<int64_t>(tgt) * cs;
+  T acc[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j) acc[j] = T(0);
+  // every lane stays in the loop to the wave's last round (the matrix
+  // instructions, the wave-wide vote and the reduction inside need the whole
+  // wave); lanes past the list repeat the target's first pair and drop the result
+  const int rounds = (e - b + kWave - 1) / kWave;
+  bool stored = ACC;  // the row holds sums already (uniform)
+  for (int q = 0; q < rounds; ++q) {
+    const int k = b + q * kWave + lane;
+    const bool live = k < e;
+    const int src = far_src[live ? k : b];
+    const V4<T> cs4 = load4(centers4, src);
+    T v[C];
+    load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
+    const T dx = ct.x - cs4.x, dy = ct.y - cs4.y, dz = ct.z - cs4.z;  // target - source
+    if constexpr (!MF && G <= kDirectM2L) {
+      // the contributions go straight into the running sums: a dead lane has a
+      // zero multipole, and sums in the way of a rescaled round are stored first
+      if (!live) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) v[j] = T(0);
+      }
+      m2l_direct_add<T, G>(v, acc, dx, dy, dz, [&] {
+        if (q == 0) return;
+        if (stored)
+          reduce_lanes<T, C, true>(acc, red, row, lane);
+        else
+          reduce_lanes<T, C, false>(acc, red, row, lane);
+        stored = true;
+#pragma unroll
+        for (int j = 0; j < C; ++j) acc[j] = T(0);
+      });
+    } else {
+      T w[C];
+      m2l_pair<T, G, MF>(v, w, dx, dy, dz, bu);
+      if (live) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) acc[j] += w[j];
+      }
+    }
+  }
+  if (stored)
+    reduce_lanes<T, C, true>(acc, red, row, lane);
+  else
+    reduce_lanes<T, C, false>(acc, red, row, lane);
   if (!ACC)
     for (int j = C + lane; j < cs; j += kWave) row[j] = T(0);
 }

@@ -13,6 +13,7 @@
 #include "device_math.hpp"
 #include "launch.hpp"
 #include "rows.hpp"
+#include "translate.hpp"
 
 namespace jfm {
 namespace {
@@ -215,15 +216,12 @@ __device__ __forceinline__ void l2l_node(int node, const int32_t* __restrict__ p
   const V4<T> cc = load4(centers4, node);
   T v[C];
   load_row<T, C>(locals + static_cast<int64_t>(par) * cs, v);
-  Align<T, P> a;
-  a.init(cp.x - cc.x, cp.y - cc.y, cp.z - cc.z);  // source(parent) - destination(child)
-  rotate_all<T, P, Rot::ToZLocal>(v, a);
-  zshift_l2l<T, P>(v, a.r);
-  rotate_all<T, P, Rot::FromZLocal>(v, a);
+  T u[C];
+  l2l<T, P>(v, u, cp.x - cc.x, cp.y - cc.y, cp.z - cc.z);  // source(parent) - destination(child)
   T w[C];
   load_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
 #pragma unroll
-  for (int j = 0; j < C; ++j) w[j] += v[j];
+  for (int j = 0; j < C; ++j) w[j] += u[j];
   store_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
 }
 
@@ -265,15 +263,12 @@ __global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ 
   const V4<T> cc = side == 0 ? cl : cr;
   T v[C];
   load_row<T, C>(mult + static_cast<int64_t>(ch) * cs, v);
-  Align<T, P> a;
-  a.init(cc.x - cx, cc.y - cy, cc.z - cz);  // source - destination
-  rotate_all<T, P, Rot::ToZMultipole>(v, a);
-  zshift_m2m<T, P>(v, a.r);
-  rotate_all<T, P, Rot::FromZMultipole>(v, a);
+  T w[C];
+  m2m<T, P>(v, w, cc.x - cx, cc.y - cy, cc.z - cz);  // source - destination
 #pragma unroll
-  for (int j = 0; j < C; ++j) v[j] = v[j] + dpp_get<0xB1>(v[j]);  // left + right on both lanes
+  for (int j = 0; j < C; ++j) w[j] = w[j] + dpp_get<0xB1>(w[j]);  // left + right on both lanes
   if (side == 0 && live) {
-    store_row<T, C>(mult + static_cast<int64_t>(node) * cs, v);
+    store_row<T, C>(mult + static_cast<int64_t>(node) * cs, w);
     store4(centers4, node, V4<T>{cx, cy, cz, tot});
   }
 }
@@ -399,20 +394,17 @@ __global__ __launch_bounds__(kWave) void m2m_top_kernel(const int32_t* __restric
 #pragma unroll
         for (int j = 0; j < C; ++j) v[j] = tmp[j];
       }
-      Align<double, P> a;
-      a.init(cc.x - cx, cc.y - cy, cc.z - cz);  // source - destination
-      rotate_all<double, P, Rot::ToZMultipole>(v, a);
-      zshift_m2m<double, P>(v, a.r);
-      rotate_all<double, P, Rot::FromZMultipole>(v, a);
+      double w[C];
+      m2m<double, P>(v, w, cc.x - cx, cc.y - cy, cc.z - cz);  // source - destination
 #pragma unroll
-      for (int j = 0; j < C; ++j) v[j] = v[j] + dpp_get<0xB1>(v[j]);  // left + right on both lanes
+      for (int j = 0; j < C; ++j) w[j] = w[j] + dpp_get<0xB1>(w[j]);  // left + right on both lanes
       if (side == 0) {
         const int sn = shadow[node];
-        store_row<double, C>(mult64 + static_cast<int64_t>(sn) * cs64, v);
+        store_row<double, C>(mult64 + static_cast<int64_t>(sn) * cs64, w);
         store4(centers64, sn, V4<double>{cx, cy, cz, tot});
         float vf[C];
 #pragma unroll
-        for (int j = 0; j < C; ++j) vf[j] = static_cast<float>(v[j]);
+        for (int j = 0; j < C; ++j) vf[j] = static_cast<float>(w[j]);
         store_row<float, C>(mult + static_cast<int64_t>(node) * cs, vf);
         store4(centers4, node, V4<float>{static_cast<float>(cx), static_cast<float>(cy), static_cast<float>(cz),
                                          static_cast<float>(tot)});
@@ -462,17 +454,16 @@ __global__ __launch_bounds__(kWave) void l2l_top_kernel(const int32_t* __restric
         const V4<float> f = load4(centers4, node);
         cn = V4<double>{f.x, f.y, f.z, f.w};
       }
-      double v[C];
-      load_row<double, C>(loc64 + static_cast<int64_t>(sp) * cs64, v);
-      Align<double, P> a;
-      a.init(cp.x - cn.x, cp.y - cn.y, cp.z - cn.z);
-      rotate_all<double, P, Rot::ToZLocal>(v, a);
-      zshift_l2l<double, P>(v, a.r);
-      rotate_all<double, P, Rot::FromZLocal>(v, a);
+      double u[C];
+      {
+        double v[C];
+        load_row<double, C>(loc64 + static_cast<int64_t>(sp) * cs64, v);
+        l2l<double, P>(v, u, cp.x - cn.x, cp.y - cn.y, cp.z - cn.z);
+      }
       if (sn >= 0) {
         double w[C];
         load_row<double, C>(loc64 + static_cast<int64_t>(sn) * cs64, w);
-        for (int j = 0; j < C; ++j) w[j] += v[j];
+        for (int j = 0; j < C; ++j) w[j] += u[j];
         store_row<double, C>(loc64 + static_cast<int64_t>(sn) * cs64, w);
         float wf[C];
         for (int j = 0; j < C; ++j) wf[j] = static_cast<float>(w[j]);
@@ -480,7 +471,7 @@ __global__ __launch_bounds__(kWave) void l2l_top_kernel(const int32_t* __restric
       } else {
         float w[C];
         load_row<float, C>(locals + static_cast<int64_t>(node) * cs, w);
-        for (int j = 0; j < C; ++j) w[j] = static_cast<float>(static_cast<double>(w[j]) + v[j]);
+        for (int j = 0; j < C; ++j) w[j] = static_cast<float>(static_cast<double>(w[j]) + u[j]);
         store_row<float, C>(locals + static_cast<int64_t>(node) * cs, w);
       }
     }
