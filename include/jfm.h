@@ -138,6 +138,11 @@ int32_t jfm_tree_leaf_geometry(void* stream, int32_t L, int32_t I, const double*
 int32_t jfm_tree_level_geometry(void* stream, int32_t count, const int32_t* level_nodes, const double* pos,
                                 const double* mass, const int32_t* perm, const int32_t* left, const int32_t* right,
                                 const int32_t* node_range, double* node_mass, double* center);
+
+/* Every level (deepest first) of jfm_tree_level_geometry, as jfm_m2m_pass. */
+int32_t jfm_tree_geometry_pass(void* stream, const int32_t* lev_off_host, int32_t nlev, const int32_t* level_nodes,
+                               const double* pos, const double* mass, const int32_t* perm, const int32_t* left,
+                               const int32_t* right, const int32_t* node_range, double* node_mass, double* center);
 /* radius [nodes] = max distance from the centre to the node's particles;
  * scratch holds n * 3 doubles (the positions in tree order). */
 int32_t jfm_tree_radius(void* stream, int32_t nodes, int64_t n, const double* pos, const int32_t* perm,
@@ -217,6 +222,15 @@ int32_t jfm_m2m_level(void* stream, int32_t dtype, int32_t p, const int32_t* nod
                       const int32_t* left, const int32_t* right, const int32_t* node_range, void* multipoles,
                       void* centers4);
 
+/* Every level of the upward pass, in order: level l holds nodes
+ * [lev_off_host[l], lev_off_host[l + 1]) of the level-ordered list `nodes`
+ * (deepest first; lev_off_host is host memory, read before the call returns).
+ * The same rows as one jfm_m2m_level per level; runs of small levels share a
+ * launch. */
+int32_t jfm_m2m_pass(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, const int32_t* lev_off_host,
+                     int32_t nlev, const int32_t* left, const int32_t* right, const int32_t* node_range,
+                     void* multipoles, void* centers4);
+
 /* M2L over the far list: locals[t] = sum_{s in far(t)} m2l(M[s], c_t - c_s) for
  * every t in targets[num_targets] (written, not accumulated; other rows untouched).
  * Replaces _apply_m2l + _accumulate_m2l_* (runtime/kernels/_m2l.py:1439-1793) and
@@ -270,6 +284,10 @@ int32_t jfm_m2l_flat(void* stream, int32_t dtype, int32_t p, int32_t gear, int32
  * Replaces _propagate_solidfmm_locals_by_level (runtime/kernels/_l2l.py:210-409). */
 int32_t jfm_l2l_level(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, int32_t count,
                       const int32_t* parent, const void* centers4, void* locals);
+
+/* Every level of the downward pass (shallowest first), as jfm_m2m_pass. */
+int32_t jfm_l2l_pass(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, const int32_t* lev_off_host,
+                     int32_t nlev, const int32_t* parent, const void* centers4, void* locals);
 
 /* Mixed precision, top three levels (float32 arrays + float64 shadows).
  * shadow[nodes] maps each internal node of depth <= 2 to its shadow row
@@ -538,6 +556,10 @@ int32_t jfm_mutual_rungs(void* stream, int32_t n, int32_t num_leaves, int32_t le
                          const int32_t* rung, int32_t* rung_sorted, int32_t* node_rung);
 int32_t jfm_mutual_rungs_level(void* stream, const int32_t* nodes, int32_t count, const int32_t* left,
                                const int32_t* right, int32_t* node_rung);
+
+/* Every level (deepest first) of jfm_mutual_rungs_level, as jfm_m2m_pass. */
+int32_t jfm_mutual_rungs_pass(void* stream, const int32_t* nodes, const int32_t* lev_off_host, int32_t nlev,
+                              const int32_t* left, const int32_t* right, int32_t* node_rung);
 /* Near-field forces F_i = G sum_j m_i m_j w[max(r_i, r_j)] (x_j - x_i) /
  * (|x_j - x_i|^2 + eps2)^{3/2} over the self leaf (j != i) and the near
  * leaves; each pair term is the exact negative of its mirror (j, i) to the

@@ -28,7 +28,7 @@ MAX_ORDER = 8
 M2L_VALU = 0
 M2L_MFMA = 1
 M2L_ENGINES = {"valu": M2L_VALU, "mfma": M2L_MFMA}
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _i32p = POINTER(c_int32)
 _f64p = POINTER(c_double)
@@ -75,6 +75,10 @@ _SIGNATURES = {
     "jfm_gather_sorted": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p]),
     "jfm_p2m": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p,
                           c_void_p]),
+    "jfm_m2m_pass": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32] + [c_void_p] * 5),
+    "jfm_l2l_pass": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32] + [c_void_p] * 3),
+    "jfm_mutual_rungs_pass": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
+    "jfm_tree_geometry_pass": (c_int32, [c_void_p, c_void_p, c_int32] + [c_void_p] * 9),
     "jfm_m2m_level": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_void_p]),
     "jfm_m2l": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -217,6 +221,13 @@ def call(name: str, *args) -> int:
                     "jfm_key_bits", "jfm_m2l_engine", "jfm_direct_sum_f64_static_max_targets"):
         check(rc, name)
     return rc
+
+
+def host_i32(a):
+    """``a`` as a contiguous int32 numpy array (no copy where it is one already)."""
+    import numpy as np
+
+    return np.ascontiguousarray(a, np.int32)
 
 
 def ptr(t) -> int | None:

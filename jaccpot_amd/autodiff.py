@@ -184,13 +184,10 @@ def fmm_vjp(fmm, state, positions: torch.Tensor, masses: torch.Tensor, acc_bar: 
              topo.num_internal, state.locals.data_ptr(), state.centers4.data_ptr(), state.G, grad_l4.data_ptr(),
              lbar.data_ptr())
     # cotangents of the locals up the tree (l2l^T = m2m on parity-flipped rows)
-    off = topo.m2m_off
-    for lev in range(len(off) - 1):
-        a, b = int(off[lev]), int(off[lev + 1])
-        if b > a:
-            nat.call("jfm_m2m_level", s, code, state.order, state.m2m_nodes.data_ptr() + 4 * a, b - a,
-                     state.left.data_ptr(), state.right.data_ptr(), state.node_range.data_ptr(), lbar.data_ptr(),
-                     state.centers4.data_ptr())
+    off = nat.host_i32(topo.m2m_off)
+    nat.call("jfm_m2m_pass", s, code, state.order, state.m2m_nodes.data_ptr(), nat.ptr(off), len(off) - 1,
+             state.left.data_ptr(), state.right.data_ptr(), state.node_range.data_ptr(), lbar.data_ptr(),
+             state.centers4.data_ptr())
     mbar = torch.zeros_like(state.multipoles)
     cbar4 = torch.zeros((topo.num_nodes, 4), dtype=dt, device=dev)
     if topo.m2l_targets.size:
@@ -212,12 +209,9 @@ def fmm_vjp(fmm, state, positions: torch.Tensor, masses: torch.Tensor, acc_bar: 
                      state.multipoles.data_ptr(), lown.data_ptr(), lbar.data_ptr(), mbar.data_ptr(),
                      state.centers4.data_ptr(), cbar4.data_ptr())
     # cotangents of the multipoles down the tree (m2m^T = l2l on parity-flipped rows)
-    off = topo.l2l_off
-    for lev in range(len(off) - 1):
-        a, b = int(off[lev]), int(off[lev + 1])
-        if b > a:
-            nat.call("jfm_l2l_level", s, code, state.order, state.l2l_nodes.data_ptr() + 4 * a, b - a,
-                     state.parent.data_ptr(), state.centers4.data_ptr(), mbar.data_ptr())
+    off = nat.host_i32(topo.l2l_off)
+    nat.call("jfm_l2l_pass", s, code, state.order, state.l2l_nodes.data_ptr(), nat.ptr(off), len(off) - 1,
+             state.parent.data_ptr(), state.centers4.data_ptr(), mbar.data_ptr())
     chain = torch.empty((topo.num_leaves, 8), dtype=dt, device=dev)
     nat.call("jfm_com_chain", s, code, topo.num_leaves, topo.num_internal, state.parent.data_ptr(),
              state.node_range.data_ptr(), state.centers4.data_ptr(), cbar4.data_ptr(), chain.data_ptr())

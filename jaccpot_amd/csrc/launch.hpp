@@ -17,6 +17,48 @@ inline int32_t check_launch(const char* what) {
   return JFM_OK;
 }
 
+// Consecutive levels of a tree sweep: offsets into the level-ordered node list,
+// passed by value.
+constexpr int kMaxSpan = 64;
+struct LevelSpan {
+  int32_t n;  // levels
+  int32_t off[kMaxSpan + 1];
+};
+
+// Walks the levels of a sweep in order: `span(LevelSpan)` for runs of two or more
+// consecutive levels of at most `small` nodes (at most kMaxSpan levels at a time),
+// `level(first node, count)` for every other level.  Empty levels are skipped.
+template <typename Span, typename Level>
+inline void for_level_spans(const int32_t* off, int32_t nlev, int32_t small, Span span, Level level) {
+  LevelSpan sp;
+  sp.n = 0;
+  auto flush = [&] {
+    if (sp.n == 1) level(sp.off[0], sp.off[1] - sp.off[0]);
+    if (sp.n > 1) span(sp);
+    sp.n = 0;
+  };
+  for (int32_t l = 0; l < nlev; ++l) {
+    const int32_t a = off[l], count = off[l + 1] - a;
+    if (count <= 0) continue;
+    if (count > small) {
+      flush();
+      level(a, count);
+      continue;
+    }
+    if (sp.n == kMaxSpan) flush();
+    if (sp.n == 0) sp.off[0] = a;
+    sp.off[++sp.n] = a + count;
+  }
+  flush();
+}
+
+inline bool valid_levels(const int32_t* off, int32_t nlev) {
+  if (nlev < 0 || (nlev > 0 && !off)) return false;
+  for (int32_t l = 0; l < nlev; ++l)
+    if (off[l + 1] < off[l] || off[l] < 0) return false;
+  return true;
+}
+
 inline bool valid_dtype(int32_t d) { return d == JFM_F32 || d == JFM_F64; }
 
 }  // namespace jfm

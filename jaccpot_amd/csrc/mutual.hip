@@ -63,6 +63,24 @@ __global__ __launch_bounds__(256) void node_rungs_kernel(const int32_t* __restri
   node_rung[u] = max(node_rung[left[u]], node_rung[right[u]]);
 }
 
+// A run of small levels in one workgroup, a barrier between the levels.
+constexpr int kRungSpanThreads = 1024;
+constexpr int kRungSpanNodes = 8 * kRungSpanThreads;
+
+__global__ __launch_bounds__(kRungSpanThreads) void node_rungs_span_kernel(const int32_t* __restrict__ nodes,
+                                                                           LevelSpan span,
+                                                                           const int32_t* __restrict__ left,
+                                                                           const int32_t* __restrict__ right,
+                                                                           int32_t* __restrict__ node_rung) {
+  for (int lev = 0; lev < span.n; ++lev) {
+    for (int k = span.off[lev] + threadIdx.x; k < span.off[lev + 1]; k += kRungSpanThreads) {
+      const int u = nodes[k];
+      node_rung[u] = max(node_rung[left[u]], node_rung[right[u]]);
+    }
+    __syncthreads();
+  }
+}
+
 // r2^(-3/2); with SAFE, 0 for r2 <= 0 (no softening: the self pair and a
 // zero-mass slot at a target's own position).  float32: v_rsq_f32 (about
 // 1 ulp) cubed.  float64: the v_rsq_f64 estimate y refined in the cube
@@ -425,6 +443,23 @@ int32_t jfm_mutual_rungs_level(void* stream, const int32_t* nodes, int32_t count
   if (!nodes || !left || !right || !node_rung) return fail(JFM_ERR_ARG, "jfm_mutual_rungs_level: NULL buffer");
   node_rungs_kernel<<<nblocks(count, 256), 256, 0, as_stream(stream)>>>(nodes, count, left, right, node_rung);
   return check_launch("jfm_mutual_rungs_level");
+}
+
+int32_t jfm_mutual_rungs_pass(void* stream, const int32_t* nodes, const int32_t* lev_off_host, int32_t nlev,
+                              const int32_t* left, const int32_t* right, int32_t* node_rung) {
+  if (!valid_levels(lev_off_host, nlev)) return fail(JFM_ERR_ARG, "jfm_mutual_rungs_pass: bad level table");
+  if (nlev == 0 || lev_off_host[nlev] == lev_off_host[0]) return JFM_OK;
+  if (!nodes || !left || !right || !node_rung) return fail(JFM_ERR_ARG, "jfm_mutual_rungs_pass: NULL buffer");
+  hipStream_t s = as_stream(stream);
+  for_level_spans(
+      lev_off_host, nlev, kRungSpanNodes,
+      [&](const LevelSpan& sp) {
+        node_rungs_span_kernel<<<1, kRungSpanThreads, 0, s>>>(nodes, sp, left, right, node_rung);
+      },
+      [&](int32_t a, int32_t count) {
+        node_rungs_kernel<<<nblocks(count, 256), 256, 0, s>>>(nodes + a, count, left, right, node_rung);
+      });
+  return check_launch("jfm_mutual_rungs_pass");
 }
 
 int32_t jfm_mutual_p2p(void* stream, int32_t dtype, const void* pos4, int32_t n, int32_t num_leaves,

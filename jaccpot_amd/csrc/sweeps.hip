@@ -204,8 +204,6 @@ __global__ __launch_bounds__(kWave) void p2m_group_kernel(const T* __restrict__ 
   if (sub == 0) store4(centers4, node, V4<T>{cx, cy, cz, ms});
 }
 
-// One thread per internal node of a level: centre of mass of the two children,
-// M = m2m(M_left, c_left - c) + m2m(M_right, c_right - c).
 // L2L into one node: L += l2l(L_parent, c_parent - c).
 template <typename T, int P>
 __device__ __forceinline__ void l2l_node(int node, const int32_t* __restrict__ parent,
@@ -225,24 +223,16 @@ __device__ __forceinline__ void l2l_node(int node, const int32_t* __restrict__ p
   store_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
 }
 
-// Two lanes per internal node of a level (children already done): lane 2i
-// translates the left child's multipole to the node's centre of mass, lane
-// 2i+1 the right one's; the sum is formed as left + right and the even lane
-// writes the node.  Halves the dependent instruction chain of a level, which
-// is what a level of the upward pass waits for.
+// Two lanes per internal node of a level (children already done): the lane of
+// side 0 translates the left child's multipole to the node's centre of mass, the
+// lane of side 1 (its neighbour t ^ 1) the right one's; the sum is formed as
+// left + right and side 0 writes the node.  Halves the dependent instruction
+// chain of a level, which is what a level of the upward pass waits for.
 template <typename T, int P>
-__global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ nodes, int32_t count,
-                                                    const int32_t* __restrict__ left,
-                                                    const int32_t* __restrict__ right,
-                                                    const int32_t* __restrict__ node_range, T* __restrict__ mult,
-                                                    int32_t cs, T* __restrict__ centers4) {
+__device__ __forceinline__ void m2m_node(int node, int side, bool live, const int32_t* __restrict__ left,
+                                         const int32_t* __restrict__ right, const int32_t* __restrict__ node_range,
+                                         T* __restrict__ mult, int32_t cs, T* __restrict__ centers4) {
   constexpr int C = ncoef(P);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int side = t & 1;
-  // lanes past the level repeat its last node (results dropped) so that both
-  // lanes of every pair reach the exchange below
-  const bool live = (t >> 1) < count;
-  const int node = nodes[live ? (t >> 1) : count - 1];
   const int lc = left[node], rc = right[node];
   const V4<T> cl = load4(centers4, lc);
   const V4<T> cr = load4(centers4, rc);
@@ -272,6 +262,59 @@ __global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ 
     store4(centers4, node, V4<T>{cx, cy, cz, tot});
   }
 }
+
+template <typename T, int P>
+__global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ nodes, int32_t count,
+                                                    const int32_t* __restrict__ left,
+                                                    const int32_t* __restrict__ right,
+                                                    const int32_t* __restrict__ node_range, T* __restrict__ mult,
+                                                    int32_t cs, T* __restrict__ centers4) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  // lanes past the level repeat its last node (results dropped) so that both
+  // lanes of every pair reach the exchange
+  const bool live = (t >> 1) < count;
+  m2m_node<T, P>(nodes[live ? (t >> 1) : count - 1], t & 1, live, left, right, node_range, mult, cs, centers4);
+}
+
+// A run of levels with few nodes each in one workgroup, a barrier between the
+// levels: such a level is one node's dependent chain (loads, about 300 VALU
+// instructions at order 4) on a nearly empty GPU, and as a launch of its own it
+// also pays the start and drain of a kernel and the host's call.  256 threads,
+// one wave per SIMD, so that the workgroup finds room on a CU beside the P2P's
+// workgroups (wider ones wait for several of those to end).
+constexpr int kSpanThreads = 256;
+
+template <typename T, int P>
+__global__ __launch_bounds__(kSpanThreads) void m2m_span_kernel(const int32_t* __restrict__ nodes, LevelSpan span,
+                                                                const int32_t* __restrict__ left,
+                                                                const int32_t* __restrict__ right,
+                                                                const int32_t* __restrict__ node_range,
+                                                                T* __restrict__ mult, int32_t cs,
+                                                                T* __restrict__ centers4) {
+  for (int lev = 0; lev < span.n; ++lev) {
+    const int b = span.off[lev], e = span.off[lev + 1];
+    for (int k = b + (threadIdx.x >> 1); k < e; k += kSpanThreads / 2)  // both lanes of a pair stay together
+      m2m_node<T, P>(nodes[k], threadIdx.x & 1, true, left, right, node_range, mult, cs, centers4);
+    __syncthreads();
+  }
+}
+
+// The same for the downward pass, one thread per node.
+template <typename T, int P>
+__global__ __launch_bounds__(kSpanThreads) void l2l_span_kernel(const int32_t* __restrict__ nodes, LevelSpan span,
+                                                                const int32_t* __restrict__ parent,
+                                                                const T* __restrict__ centers4,
+                                                                T* __restrict__ locals, int32_t cs) {
+  for (int lev = 0; lev < span.n; ++lev) {
+    for (int k = span.off[lev] + threadIdx.x; k < span.off[lev + 1]; k += kSpanThreads)
+      l2l_node<T, P>(nodes[k], parent, centers4, locals, cs);
+    __syncthreads();
+  }
+}
+
+// Levels of at most this many nodes join a span: SPAN_ROUNDS passes of the
+// workgroup over a level, which then costs about as much as a launch.
+constexpr int span_rounds(int p) { return p <= 4 ? 2 : 1; }
 
 // One thread per node of a level: L += l2l(L_parent, c_parent - c).
 template <typename T, int P>
@@ -571,6 +614,51 @@ int32_t jfm_l2l_level(void* stream, int32_t dtype, int32_t p, const int32_t* nod
                                                                 (T*)locals, cs);
   }));
   return check_launch("jfm_l2l_level");
+}
+
+int32_t jfm_m2m_pass(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, const int32_t* lev_off_host,
+                     int32_t nlev, const int32_t* left, const int32_t* right, const int32_t* node_range,
+                     void* multipoles, void* centers4) {
+  if (!valid_levels(lev_off_host, nlev)) return fail(JFM_ERR_ARG, "jfm_m2m_pass: bad level table");
+  if (nlev == 0 || lev_off_host[nlev] == lev_off_host[0]) return JFM_OK;
+  if (!nodes || !left || !right || !node_range || !multipoles || !centers4)
+    return fail(JFM_ERR_ARG, "jfm_m2m_pass: NULL buffer");
+  hipStream_t s = as_stream(stream);
+  JFM_FOR_DTYPE(dtype, JFM_FOR_ORDER(p, {
+    const int cs = coef_stride(P, sizeof(T));
+    for_level_spans(
+        lev_off_host, nlev, span_rounds(P) * kSpanThreads / 2,
+        [&](const LevelSpan& sp) {
+          m2m_span_kernel<T, P><<<1, kSpanThreads, 0, s>>>(nodes, sp, left, right, node_range, (T*)multipoles, cs,
+                                                           (T*)centers4);
+        },
+        [&](int32_t a, int32_t count) {
+          m2m_kernel<T, P><<<blocks_for(2 * static_cast<int64_t>(count), kWave), kWave, 0, s>>>(
+              nodes + a, count, left, right, node_range, (T*)multipoles, cs, (T*)centers4);
+        });
+  }));
+  return check_launch("jfm_m2m_pass");
+}
+
+int32_t jfm_l2l_pass(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, const int32_t* lev_off_host,
+                     int32_t nlev, const int32_t* parent, const void* centers4, void* locals) {
+  if (!valid_levels(lev_off_host, nlev)) return fail(JFM_ERR_ARG, "jfm_l2l_pass: bad level table");
+  if (nlev == 0 || lev_off_host[nlev] == lev_off_host[0]) return JFM_OK;
+  if (!nodes || !parent || !centers4 || !locals) return fail(JFM_ERR_ARG, "jfm_l2l_pass: NULL buffer");
+  hipStream_t s = as_stream(stream);
+  JFM_FOR_DTYPE(dtype, JFM_FOR_ORDER(p, {
+    const int cs = coef_stride(P, sizeof(T));
+    for_level_spans(
+        lev_off_host, nlev, span_rounds(P) * kSpanThreads,
+        [&](const LevelSpan& sp) {
+          l2l_span_kernel<T, P><<<1, kSpanThreads, 0, s>>>(nodes, sp, parent, (const T*)centers4, (T*)locals, cs);
+        },
+        [&](int32_t a, int32_t count) {
+          l2l_kernel<T, P><<<blocks_for(count, kWave), kWave, 0, s>>>(nodes + a, count, parent, (const T*)centers4,
+                                                                      (T*)locals, cs);
+        });
+  }));
+  return check_launch("jfm_l2l_pass");
 }
 
 int32_t jfm_m2m_top(void* stream, int32_t p, const int32_t* nodes, const int32_t* lev_off, int32_t nlev,

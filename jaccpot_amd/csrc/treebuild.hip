@@ -265,16 +265,9 @@ __global__ void __launch_bounds__(256) leaf_geometry_kernel(Particles P, int32_t
   }
 }
 
-__global__ void __launch_bounds__(256) internal_geometry_kernel(Particles P, int32_t count,
-                                                                const int32_t* __restrict__ level_nodes,
-                                                                const int32_t* __restrict__ left,
-                                                                const int32_t* __restrict__ right,
-                                                                const int32_t* __restrict__ range,
-                                                                double* __restrict__ mass,
-                                                                double* __restrict__ center) {
-  const int32_t q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= count) return;
-  const int32_t node = level_nodes[q];
+__device__ inline void internal_geometry(Particles P, int32_t node, const int32_t* __restrict__ left,
+                                         const int32_t* __restrict__ right, const int32_t* __restrict__ range,
+                                         double* __restrict__ mass, double* __restrict__ center) {
   const int32_t lc = left[node], rc = right[node];
   const double ml = mass[lc], mr = mass[rc];
   const double tot = ml + mr;
@@ -283,6 +276,32 @@ __global__ void __launch_bounds__(256) internal_geometry_kernel(Particles P, int
     for (int k = 0; k < 3; ++k) center[3 * node + k] = (ml * center[3 * lc + k] + mr * center[3 * rc + k]) / tot;
   } else {
     mean_of(P, range[2 * node], range[2 * node + 1], &center[3 * node]);
+  }
+}
+
+__global__ void __launch_bounds__(256) internal_geometry_kernel(Particles P, int32_t count,
+                                                                const int32_t* __restrict__ level_nodes,
+                                                                const int32_t* __restrict__ left,
+                                                                const int32_t* __restrict__ right,
+                                                                const int32_t* __restrict__ range,
+                                                                double* __restrict__ mass,
+                                                                double* __restrict__ center) {
+  const int32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q < count) internal_geometry(P, level_nodes[q], left, right, range, mass, center);
+}
+
+// A run of small levels in one workgroup, a barrier between the levels.
+constexpr int kGeometrySpanThreads = 512;
+constexpr int kGeometrySpanNodes = 2 * kGeometrySpanThreads;
+
+__global__ void __launch_bounds__(kGeometrySpanThreads) internal_geometry_span_kernel(
+    Particles P, LevelSpan span, const int32_t* __restrict__ level_nodes, const int32_t* __restrict__ left,
+    const int32_t* __restrict__ right, const int32_t* __restrict__ range, double* __restrict__ mass,
+    double* __restrict__ center) {
+  for (int lev = 0; lev < span.n; ++lev) {
+    for (int k = span.off[lev] + threadIdx.x; k < span.off[lev + 1]; k += kGeometrySpanThreads)
+      internal_geometry(P, level_nodes[k], left, right, range, mass, center);
+    __syncthreads();
   }
 }
 
@@ -574,6 +593,28 @@ int32_t jfm_tree_level_geometry(void* stream, int32_t count, const int32_t* leve
   hipLaunchKernelGGL(jfm::internal_geometry_kernel, dim3(jfm::grid_for(count)), dim3(256), 0, jfm::as_stream(stream),
                      P, count, level_nodes, left, right, node_range, node_mass, center);
   return jfm::check_launch("jfm_tree_level_geometry");
+}
+
+int32_t jfm_tree_geometry_pass(void* stream, const int32_t* lev_off_host, int32_t nlev, const int32_t* level_nodes,
+                               const double* pos, const double* mass, const int32_t* perm, const int32_t* left,
+                               const int32_t* right, const int32_t* node_range, double* node_mass, double* center) {
+  if (!jfm::valid_levels(lev_off_host, nlev)) return fail(JFM_ERR_ARG, "jfm_tree_geometry_pass: bad level table");
+  if (nlev == 0 || lev_off_host[nlev] == lev_off_host[0]) return JFM_OK;
+  if (!level_nodes || !pos || !mass || !perm || !left || !right || !node_range || !node_mass || !center)
+    return fail(JFM_ERR_ARG, "jfm_tree_geometry_pass: bad argument");
+  jfm::Particles P{pos, mass, perm};
+  hipStream_t s = jfm::as_stream(stream);
+  jfm::for_level_spans(
+      lev_off_host, nlev, jfm::kGeometrySpanNodes,
+      [&](const jfm::LevelSpan& sp) {
+        hipLaunchKernelGGL(jfm::internal_geometry_span_kernel, dim3(1), dim3(jfm::kGeometrySpanThreads), 0, s, P, sp,
+                           level_nodes, left, right, node_range, node_mass, center);
+      },
+      [&](int32_t a, int32_t count) {
+        hipLaunchKernelGGL(jfm::internal_geometry_kernel, dim3(jfm::grid_for(count)), dim3(256), 0, s, P, count,
+                           level_nodes + a, left, right, node_range, node_mass, center);
+      });
+  return jfm::check_launch("jfm_tree_geometry_pass");
 }
 
 int32_t jfm_tree_radius(void* stream, int32_t nodes, int64_t n, const double* pos, const int32_t* perm,

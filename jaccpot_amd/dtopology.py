@@ -177,12 +177,10 @@ def build_topology_device(x: torch.Tensor, m: torch.Tensor, *, leaf_size: int, t
     radius = torch.empty(nodes, dtype=torch.float64, device=dev)
     nat.call("jfm_tree_leaf_geometry", s, L, I, x.data_ptr(), m.data_ptr(), perm.data_ptr(), node_range.data_ptr(),
              mass.data_ptr(), center.data_ptr())
-    for lev in range(len(m2m_off) - 1):
-        a, b = int(m2m_off[lev]), int(m2m_off[lev + 1])
-        if b > a:
-            nat.call("jfm_tree_level_geometry", s, b - a, m2m_nodes[a:].data_ptr(), x.data_ptr(), m.data_ptr(),
-                     perm.data_ptr(), left.data_ptr(), right.data_ptr(), node_range.data_ptr(), mass.data_ptr(),
-                     center.data_ptr())
+    m2m_off = nat.host_i32(m2m_off)
+    nat.call("jfm_tree_geometry_pass", s, nat.ptr(m2m_off), len(m2m_off) - 1, m2m_nodes.data_ptr(), x.data_ptr(),
+             m.data_ptr(), perm.data_ptr(), left.data_ptr(), right.data_ptr(), node_range.data_ptr(), mass.data_ptr(),
+             center.data_ptr())
     xs = torch.empty((n, 3), dtype=torch.float64, device=dev)
     nat.call("jfm_tree_radius", s, nodes, n, x.data_ptr(), perm.data_ptr(), node_range.data_ptr(), center.data_ptr(),
              xs.data_ptr(), radius.data_ptr())

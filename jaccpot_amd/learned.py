@@ -210,12 +210,10 @@ def pair_labels(state, gears: Sequence[int] = (2, 4, 6)) -> torch.Tensor:
     code = nat.JFM_F32
     nat.call("jfm_p2m", s, code, 8, state.pos4.data_ptr(), topo.num_particles, topo.num_leaves, topo.leaf_size,
              topo.num_internal, mult8.data_ptr(), centers.data_ptr())
-    off = topo.m2m_off
-    for lev in range(len(off) - 1):
-        a, b = int(off[lev]), int(off[lev + 1])
-        if b > a:
-            nat.call("jfm_m2m_level", s, code, 8, state.m2m_nodes.data_ptr() + 4 * a, b - a, state.left.data_ptr(),
-                     state.right.data_ptr(), state.node_range.data_ptr(), mult8.data_ptr(), centers.data_ptr())
+    off = nat.host_i32(topo.m2m_off)
+    nat.call("jfm_m2m_pass", s, code, 8, state.m2m_nodes.data_ptr(), nat.ptr(off), len(off) - 1,
+             state.left.data_ptr(), state.right.data_ptr(), state.node_range.data_ptr(), mult8.data_ptr(),
+             centers.data_ptr())
     tgt, src, rad = pair_arrays(state)
     T = torch.empty((K, NUM_OUTPUTS), dtype=torch.float32, device=dev)
     g3 = np.asarray(tuple(int(g) for g in gears), np.int32)

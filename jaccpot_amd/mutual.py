@@ -329,27 +329,22 @@ def _levels(st: MutualFMMState, rung, level_weights):
         raise ValueError(f"rung must have {topo.num_particles} entries")
     nat.call("jfm_mutual_rungs", s, topo.num_particles, topo.num_leaves, topo.leaf_size, prep.perm.data_ptr(),
              r.data_ptr(), st.buffers["rung_sorted"].data_ptr(), st.buffers["node_rung"].data_ptr())
-    off = st.level_off
-    for lev in range(len(off) - 1):  # deepest level first
-        a, b = int(off[lev]), int(off[lev + 1])
-        if b > a:
-            nat.call("jfm_mutual_rungs_level", s, prep.m2m_nodes.data_ptr() + 4 * a, b - a, prep.left.data_ptr(),
-                     prep.right.data_ptr(), st.buffers["node_rung"].data_ptr())
+    off = nat.host_i32(st.level_off)  # deepest level first
+    nat.call("jfm_mutual_rungs_pass", s, prep.m2m_nodes.data_ptr(), nat.ptr(off), len(off) - 1, prep.left.data_ptr(),
+             prep.right.data_ptr(), st.buffers["node_rung"].data_ptr())
     return lw
 
 
 def _tree_level(prep, nodes: torch.Tensor, off, op: str, rows: torch.Tensor, code: int, s) -> None:
     """One pass of M2M (deepest level first) or L2L (root first) over ``rows``."""
-    for lev in range(len(off) - 1):
-        a, b = int(off[lev]), int(off[lev + 1])
-        if b <= a:
-            continue
-        if op == "m2m":
-            nat.call("jfm_m2m_level", s, code, prep.order, nodes.data_ptr() + 4 * a, b - a, prep.left.data_ptr(),
-                     prep.right.data_ptr(), prep.node_range.data_ptr(), rows.data_ptr(), prep.centers4.data_ptr())
-        else:
-            nat.call("jfm_l2l_level", s, code, prep.order, nodes.data_ptr() + 4 * a, b - a, prep.parent.data_ptr(),
-                     prep.centers4.data_ptr(), rows.data_ptr())
+    off = nat.host_i32(off)
+    if op == "m2m":
+        nat.call("jfm_m2m_pass", s, code, prep.order, nodes.data_ptr(), nat.ptr(off), len(off) - 1,
+                 prep.left.data_ptr(), prep.right.data_ptr(), prep.node_range.data_ptr(), rows.data_ptr(),
+                 prep.centers4.data_ptr())
+    else:
+        nat.call("jfm_l2l_pass", s, code, prep.order, nodes.data_ptr(), nat.ptr(off), len(off) - 1,
+                 prep.parent.data_ptr(), prep.centers4.data_ptr(), rows.data_ptr())
 
 
 def _far_m2l(st: MutualFMMState, lw, src: torch.Tensor, dst: torch.Tensor, code: int, s) -> None:

@@ -517,17 +517,13 @@ class FastMultipoleMethod:
         mixed = state.extra.get("mixed")
         if p2m:
             self._p2m(state, s, code)
-        off = topo.m2m_off
-        base = state.m2m_nodes.data_ptr()
-        D = topo.max_depth
-        for lev in range(len(off) - 1):
-            a, b = int(off[lev]), int(off[lev + 1])
-            if mixed is not None and D - lev <= 2:
-                continue  # float64 top levels below
-            if b > a:
-                nat.call("jfm_m2m_level", s, code, state.order, base + 4 * a, b - a, state.left.data_ptr(),
-                         state.right.data_ptr(), state.node_range.data_ptr(), state.multipoles.data_ptr(),
-                         state.centers4.data_ptr())
+        off = nat.host_i32(topo.m2m_off)
+        nlev = len(off) - 1
+        if mixed is not None:  # level l is depth max_depth - l; depths 0..2 run in float64 below
+            nlev = min(nlev, max(topo.max_depth - 2, 0))
+        nat.call("jfm_m2m_pass", s, code, state.order, state.m2m_nodes.data_ptr(), nat.ptr(off), nlev,
+                 state.left.data_ptr(), state.right.data_ptr(), state.node_range.data_ptr(),
+                 state.multipoles.data_ptr(), state.centers4.data_ptr())
         if mixed is not None and mixed["ntop"]:
             oh = mixed["m2m_off_host"]
             nat.call("jfm_m2m_top", s, state.order, mixed["m2m_nodes"].data_ptr(), mixed["m2m_off"].data_ptr(),
@@ -575,13 +571,9 @@ class FastMultipoleMethod:
                      mixed["shadow"].data_ptr(), state.centers4.data_ptr(), mixed["centers64"].data_ptr(),
                      state.locals.data_ptr(), mixed["loc64"].data_ptr())
             first_lev = 3  # depths 1..3 done in float64
-        off = topo.l2l_off
-        base = state.l2l_nodes.data_ptr()
-        for lev in range(first_lev, len(off) - 1):
-            a, b = int(off[lev]), int(off[lev + 1])
-            if b > a:
-                nat.call("jfm_l2l_level", s, code, state.order, base + 4 * a, b - a, state.parent.data_ptr(),
-                         state.centers4.data_ptr(), state.locals.data_ptr())
+        off = nat.host_i32(topo.l2l_off[first_lev:])
+        nat.call("jfm_l2l_pass", s, code, state.order, state.l2l_nodes.data_ptr(), nat.ptr(off), max(len(off) - 1, 0),
+                 state.parent.data_ptr(), state.centers4.data_ptr(), state.locals.data_ptr())
 
     # ------------------------------------------------------------- evaluate
     def _evaluate_device(self, state: FMMPreparedState, acc: torch.Tensor, pot: Optional[torch.Tensor],
