@@ -144,21 +144,39 @@ int32_t jfm_tree_geometry_pass(void* stream, const int32_t* lev_off_host, int32_
                                const double* pos, const double* mass, const int32_t* perm, const int32_t* left,
                                const int32_t* right, const int32_t* node_range, double* node_mass, double* center);
 /* radius [nodes] = max distance from the centre to the node's particles;
- * scratch holds n * 3 doubles (the positions in tree order). */
+ * scratch holds n * 3 doubles (the positions in tree order), work 2 + 2 *
+ * work_cap int32 with work_cap >= jfm_tree_radius_work(nodes, n, max_depth). */
+int64_t jfm_tree_radius_work(int32_t nodes, int64_t n, int32_t max_depth);
 int32_t jfm_tree_radius(void* stream, int32_t nodes, int64_t n, const double* pos, const int32_t* perm,
-                        const int32_t* node_range, const double* center, double* scratch, double* radius);
-/* One breadth-first step of the dual-tree walk in three calls.  classify:
- * codes [n_in] (what item t emits) and counts3 [3][n_in] (items, far keys,
- * near keys of item t); jfm_scan_i32 on each row of counts3 gives offsets3;
- * emit: item t writes its child items at items_out[offsets3[0][t]], its far
- * pairs (target << 32 | source node) at far_keys[far_base + offsets3[1][t]]
- * and its near pairs (target << 32 | source leaf) at near_keys[near_base +
- * offsets3[2][t]] (the caller sizes every output from the scanned totals). */
-int32_t jfm_tree_walk_classify(void* stream, int32_t I, const int32_t* items_in, int64_t n_in, const double* center,
-                               const double* radius, double theta, uint8_t* codes, int32_t* counts3);
-int32_t jfm_tree_walk_emit(void* stream, int32_t I, const int32_t* items_in, int64_t n_in, const int32_t* left,
-                           const int32_t* right, const uint8_t* codes, const int32_t* offsets3, int64_t far_base,
-                           int64_t near_base, int32_t* items_out, uint64_t* far_keys, uint64_t* near_keys);
+                        const int32_t* node_range, const double* center, double* scratch, int32_t* work,
+                        int64_t work_cap, double* radius);
+/* node4 [nodes][4] = centre and radius, the record the walk reads. */
+int32_t jfm_tree_pack_nodes(void* stream, int32_t nodes, const double* center, const double* radius, void* node4);
+/* Breadth-first steps of the dual-tree walk, without a host read between them.
+ * frontier0/1: int32 pairs (a, b), frontier_cap each; the walk starts from the
+ * one item (0, 0) in frontier0.  far, near: packed keys (target << shift) |
+ * source (nodes; leaves), uint64 where wide, else uint32 (2 * shift <= 32);
+ * their order is unspecified.  state: jfm_tree_walk_state_words(steps) words,
+ * zero except word 48 = 1 (the items of the first frontier), for steps =
+ * all steps that will be launched.  One call launches `groups` groups (one
+ * workgroup that runs steps while the frontier is small, then steps_per_group
+ * steps over the whole GPU) and one more small step: steps first_step ..
+ * first_step + groups * (1 + steps_per_group).  Afterwards word 48 + 2 t holds
+ * the frontier's items before step t (0: the walk has ended), words 0 and 16
+ * the far and near keys found, word 32 which buffer was too small (1 frontier,
+ * 2 far, 4 near): keys that do not fit are counted, not written, while a full
+ * frontier ends the walk, word 33 then holding items it needed at least. */
+int32_t jfm_tree_walk_state_words(int32_t steps);
+int32_t jfm_tree_walk(void* stream, int32_t I, const void* node4, const int32_t* left, const int32_t* right,
+                      double theta, void* frontier0, void* frontier1, int64_t frontier_cap, void* far,
+                      int64_t far_cap, int32_t far_shift, int32_t far_wide, void* near, int64_t near_cap,
+                      int32_t near_shift, int32_t near_wide, uint64_t* state, int32_t first_step, int32_t groups,
+                      int32_t steps_per_group);
+/* Packed keys -> CSR off [rows+1], col [n] (columns ascending in a row);
+ * sorted [n] keys, scratch jfm_sort_packed_scratch_bytes(n, wide) bytes. */
+int32_t jfm_sort_packed_scratch_bytes(int64_t n, int32_t wide, int64_t* bytes);
+int32_t jfm_packed_to_csr(void* stream, int64_t n, int32_t wide, int32_t shift, const void* keys, void* sorted,
+                          void* scratch, int64_t scratch_bytes, int32_t rows, int32_t* off, int32_t* col);
 /* Exclusive prefix sum of int32 values; scratch holds jfm_scan_scratch_bytes(n). */
 int32_t jfm_scan_scratch_bytes(int64_t n, int64_t* bytes);
 int32_t jfm_scan_i32(void* stream, int64_t n, const int32_t* in, int32_t* out, void* scratch, int64_t scratch_bytes);

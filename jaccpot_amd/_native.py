@@ -28,7 +28,7 @@ MAX_ORDER = 8
 M2L_VALU = 0
 M2L_MFMA = 1
 M2L_ENGINES = {"valu": M2L_VALU, "mfma": M2L_MFMA}
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _i32p = POINTER(c_int32)
 _f64p = POINTER(c_double)
@@ -56,11 +56,16 @@ _SIGNATURES = {
                                   c_void_p]),
     "jfm_tree_leaf_geometry": (c_int32, [c_void_p, c_int32, c_int32] + [c_void_p] * 6),
     "jfm_tree_level_geometry": (c_int32, [c_void_p, c_int32] + [c_void_p] * 9),
-    "jfm_tree_radius": (c_int32, [c_void_p, c_int32, c_int64] + [c_void_p] * 6),
-    "jfm_tree_walk_classify": (c_int32, [c_void_p, c_int32, c_void_p, c_int64, c_void_p, c_void_p, c_double,
-                                         c_void_p, c_void_p]),
-    "jfm_tree_walk_emit": (c_int32, [c_void_p, c_int32, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
-                                     c_int64, c_int64, c_void_p, c_void_p, c_void_p]),
+    "jfm_tree_radius_work": (c_int64, [c_int32, c_int64, c_int32]),
+    "jfm_tree_radius": (c_int32, [c_void_p, c_int32, c_int64] + [c_void_p] * 6 + [c_int64, c_void_p]),
+    "jfm_tree_pack_nodes": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
+    "jfm_tree_walk_state_words": (c_int32, [c_int32]),
+    "jfm_tree_walk": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_void_p, c_int64,
+                                c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64, c_int32, c_int32, c_void_p,
+                                c_int32, c_int32, c_int32]),
+    "jfm_sort_packed_scratch_bytes": (c_int32, [c_int64, c_int32, POINTER(c_int64)]),
+    "jfm_packed_to_csr": (c_int32, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
+                                    c_void_p, c_void_p]),
     "jfm_scan_scratch_bytes": (c_int32, [c_int64, POINTER(c_int64)]),
     "jfm_scan_i32": (c_int32, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64]),
     "jfm_keys_to_csr": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
@@ -218,7 +223,7 @@ def call(name: str, *args) -> int:
     rc = getattr(load(), name)(*args)
     if name not in ("jfm_direct_scratch_doubles", "jfm_coeff_stride", "jfm_order_supported", "jfm_abi_version",
                     "jfm_mlp_num_params", "jfm_mlp_backward_scratch_floats", "jfm_tree_bounds_scratch_doubles",
-                    "jfm_key_bits", "jfm_m2l_engine", "jfm_direct_sum_f64_static_max_targets"):
+                    "jfm_key_bits", "jfm_tree_radius_work", "jfm_tree_walk_state_words", "jfm_m2l_engine", "jfm_direct_sum_f64_static_max_targets"):
         check(rc, name)
     return rc
 

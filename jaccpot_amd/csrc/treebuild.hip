@@ -19,16 +19,17 @@
 //    three child items; MAC (r_a + r_b)^2 <= theta^2 d^2, d > 0 -> far pair in
 //    both directions; two leaves -> near pair in both directions; otherwise
 //    split the larger-radius non-leaf node).  The walk's set of pairs does not
-//    depend on the expansion order; sorting the packed (target << 32 | source)
-//    keys gives the host's CSR (targets ascending, sources ascending).
+//    depend on the expansion order; sorting the packed (target, source) keys
+//    gives the host's CSR (targets ascending, sources ascending).
 //
 // Floating-point expressions are evaluated without contraction so every sum,
 // product, quotient and square root rounds exactly as the host's.
 //
 // Buffers are the caller's; the sorts and scans take a caller-provided
-// scratch (jfm_sort_scratch_bytes, jfm_scan_scratch_bytes).  A walk step is
-// classify (what each item emits), an exclusive scan of the counts, and emit
-// (each item writes at its offsets), so the caller sizes every output exactly.
+// scratch (jfm_sort_scratch_bytes, jfm_scan_scratch_bytes).  The walk's steps
+// read and leave their counts on the device, so many are launched without the
+// host looking at them; a list that does not fit its buffer is counted on and
+// reported, and the caller walks again with larger ones.
 
 #pragma clang fp contract(off)
 
@@ -306,29 +307,50 @@ __global__ void __launch_bounds__(kGeometrySpanThreads) internal_geometry_span_k
 }
 
 // tree-order copy of the positions, so the radius sweeps read contiguously
-__global__ void __launch_bounds__(256) sorted_positions_kernel(Particles P, int64_t n, double* __restrict__ xs) {
+// (and the zeroing of the radius work counter)
+__global__ void __launch_bounds__(256) sorted_positions_kernel(Particles P, int64_t n, double* __restrict__ xs,
+                                                               int32_t* __restrict__ work_count) {
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
+  if (i == 0) *work_count = 0;
   for (int a = 0; a < 3; ++a) xs[3 * i + a] = P.x(i, a);
 }
 
 constexpr int kSmallRadius = 2048;  // nodes up to this many particles: one wave each
+constexpr int kRadiusChunk = 4096;  // particles per work item of a larger node
+constexpr int kRadiusBlocks = 2048;
 
 __device__ inline double dist2(const double* __restrict__ xs, int64_t i, double cx, double cy, double cz) {
   const double dx = xs[3 * i] - cx, dy = xs[3 * i + 1] - cy, dz = xs[3 * i + 2] - cz;
   return dx * dx + dy * dy + dz * dz;
 }
 
-// one wave per node of at most kSmallRadius particles: max squared distance
+// One wave per node: a node of at most kSmallRadius particles gets its radius,
+// a larger one is cut into (node, chunk) work items for radius_big_kernel, with
+// its radius entry zeroed to hold the squared maximum's bits meanwhile.  One
+// workgroup per large node left the root and its neighbours running alone on a
+// few CUs (269 us of a 1M-body build; 40 us in chunks).
 __global__ void __launch_bounds__(256) radius_small_kernel(const double* __restrict__ xs, int32_t nodes,
                                                            const int32_t* __restrict__ range,
                                                            const double* __restrict__ center,
-                                                           double* __restrict__ radius) {
+                                                           double* __restrict__ radius, int2* __restrict__ work,
+                                                           int32_t work_cap, int32_t* __restrict__ work_count) {
   const int32_t node = blockIdx.x * 4 + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
   if (node >= nodes) return;  // whole waves leave together
   const int64_t a = range[2 * node], b = range[2 * node + 1];
-  if (b - a + 1 > kSmallRadius) return;
+  if (b - a + 1 > kSmallRadius) {
+    const int chunks = static_cast<int>((b - a + kRadiusChunk) / kRadiusChunk);
+    int at = 0;
+    if (lane == 0) {
+      radius[node] = 0.0;
+      at = atomicAdd(work_count, chunks);
+    }
+    at = __shfl(at, 0);
+    for (int c = lane; c < chunks; c += 64)
+      if (at + c < work_cap) work[at + c] = make_int2(node, c);
+    return;
+  }
   const double cx = center[3 * node], cy = center[3 * node + 1], cz = center[3 * node + 2];
   double best = 0.0;
   for (int64_t i = a + lane; i <= b; i += 64) best = fmax(best, dist2(xs, i, cx, cy, cz));
@@ -336,113 +358,256 @@ __global__ void __launch_bounds__(256) radius_small_kernel(const double* __restr
   if (lane == 0) radius[node] = sqrt(best);
 }
 
-// one 1024-thread block per larger node, four independent loads in flight per thread
-__global__ void __launch_bounds__(1024) radius_big_kernel(const double* __restrict__ xs, int32_t nodes,
-                                                          const int32_t* __restrict__ range,
-                                                          const double* __restrict__ center,
+// The larger nodes' work items, dealt to a fixed grid; the squared maxima of a
+// node's items meet by an integer maximum of their bits (order preserving for
+// non-negative doubles, so the result does not depend on the order).
+__global__ void __launch_bounds__(256) radius_big_kernel(const double* __restrict__ xs,
+                                                         const int32_t* __restrict__ range,
+                                                         const double* __restrict__ center,
+                                                         const int2* __restrict__ work, int32_t work_cap,
+                                                         const int32_t* __restrict__ work_count,
+                                                         double* __restrict__ radius) {
+  const int32_t count = min(*work_count, work_cap);
+  for (int32_t w = blockIdx.x * 4 + threadIdx.x / 64; w < count; w += gridDim.x * 4) {  // a wave per item
+    const int2 it = work[w];
+    const int64_t a = range[2 * it.x] + int64_t(it.y) * kRadiusChunk;
+    const int64_t e = min(a + kRadiusChunk - 1, int64_t(range[2 * it.x + 1]));
+    const double cx = center[3 * it.x], cy = center[3 * it.x + 1], cz = center[3 * it.x + 2];
+    double best = 0.0;
+    int64_t i = a + threadIdx.x % 64;
+    for (; i + 3 * 64 <= e; i += 4 * 64) {  // four independent loads in flight
+      const double d0 = dist2(xs, i, cx, cy, cz), d1 = dist2(xs, i + 64, cx, cy, cz);
+      const double d2 = dist2(xs, i + 128, cx, cy, cz), d3 = dist2(xs, i + 192, cx, cy, cz);
+      best = fmax(best, fmax(fmax(d0, d1), fmax(d2, d3)));
+    }
+    for (; i <= e; i += 64) best = fmax(best, dist2(xs, i, cx, cy, cz));
+    for (int off = 32; off >= 1; off >>= 1) best = fmax(best, __shfl_xor(best, off));
+    if (threadIdx.x % 64 == 0)
+      atomicMax(reinterpret_cast<unsigned long long*>(radius + it.x),
+                static_cast<unsigned long long>(__double_as_longlong(best)));
+  }
+}
+
+__global__ void __launch_bounds__(256) radius_root_kernel(int32_t nodes, const int32_t* __restrict__ range,
                                                           double* __restrict__ radius) {
-  __shared__ double red[16];
-  const int32_t node = blockIdx.x;
-  const int64_t a = range[2 * node], b = range[2 * node + 1];
-  if (b - a + 1 <= kSmallRadius) return;  // uniform per block
-  const double cx = center[3 * node], cy = center[3 * node + 1], cz = center[3 * node + 2];
-  double best = 0.0;
-  int64_t i = a + threadIdx.x;
-  for (; i + 3 * 1024 <= b; i += 4 * 1024) {
-    const double d0 = dist2(xs, i, cx, cy, cz), d1 = dist2(xs, i + 1024, cx, cy, cz);
-    const double d2 = dist2(xs, i + 2048, cx, cy, cz), d3 = dist2(xs, i + 3072, cx, cy, cz);
-    best = fmax(best, fmax(fmax(d0, d1), fmax(d2, d3)));
-  }
-  for (; i <= b; i += 1024) best = fmax(best, dist2(xs, i, cx, cy, cz));
-  for (int off = 32; off >= 1; off >>= 1) best = fmax(best, __shfl_xor(best, off));
-  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = best;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w) best = fmax(best, red[w]);
-    radius[node] = sqrt(best);
-  }
+  const int32_t node = blockIdx.x * 256 + threadIdx.x;
+  if (node < nodes && range[2 * node + 1] - range[2 * node] + 1 > kSmallRadius) radius[node] = sqrt(radius[node]);
 }
 
 // ---------------------------------------------------------------------------
-// dual-tree walk, one breadth-first step
+// dual-tree walk, breadth first
 // ---------------------------------------------------------------------------
 
-// Every frontier item is classified first (what it emits), the per-item
-// counts are exclusive-scanned, and a second pass writes each item's outputs
-// at its scanned offsets: no atomics, and the output order is a function of
-// the input order alone.
-enum WalkCode : uint8_t { kNone = 0, kSelf = 1, kFar = 2, kNear = 3, kSplitA = 4, kSplitB = 5 };
+// State of a walk on the device (int64 each; the three counters that every
+// workgroup adds to lie in cache lines of their own).
+enum WalkSlot { kFarCount = 0, kNearCount = 16, kOverflow = 32, kFrontierNeed = 33, kSteps = 48 };
+// kSteps + 2 t: items of the frontier that step t reads, + 1: the buffer it lies in.
+enum WalkFull : int { kFullFrontier = 1, kFullFar = 2, kFullNear = 4 };
 
-__global__ void __launch_bounds__(256) walk_classify_kernel(const int2* __restrict__ in, int64_t n_in, int32_t I,
-                                                            const double* __restrict__ C,
-                                                            const double* __restrict__ R, double th2,
-                                                            uint8_t* __restrict__ code,
-                                                            int32_t* __restrict__ counts3) {
-  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= n_in) return;
-  const int32_t a = in[t].x, b = in[t].y;
-  uint8_t c;
-  if (a == b) {
-    c = a < I ? kSelf : kNone;
+enum WalkCode : uint32_t { kNone = 0, kSelf = 1, kFar = 2, kNear = 3, kSplitA = 4, kSplitB = 5 };
+
+struct Walk {
+  int32_t I;
+  double th2;
+  const double4* node;  // centre and radius
+  const int32_t* left;
+  const int32_t* right;
+  int2* frontier[2];
+  int64_t frontier_cap;
+  void* far;  // packed keys (target << shift) | source, uint32 where `wide` is 0
+  int64_t far_cap;
+  int32_t far_shift, far_wide;
+  void* near;
+  int64_t near_cap;
+  int32_t near_shift, near_wide;
+  unsigned long long* st;
+};
+
+__global__ void __launch_bounds__(256) pack_nodes_kernel(int32_t nodes, const double* __restrict__ C,
+                                                         const double* __restrict__ R, double4* __restrict__ out) {
+  const int32_t k = blockIdx.x * 256 + threadIdx.x;
+  if (k < nodes) out[k] = make_double4(C[3 * k], C[3 * k + 1], C[3 * k + 2], R[k]);
+}
+
+__device__ inline uint32_t walk_code(const Walk& w, int2 it) {
+  const int32_t a = it.x, b = it.y;
+  if (a == b) return a < w.I ? kSelf : kNone;
+  const double4 A = w.node[a], B = w.node[b];
+  const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+  const double d2 = dx * dx + dy * dy + dz * dz;
+  const double s = A.w + B.w;
+  const bool al = a >= w.I, bl = b >= w.I;
+  if (d2 > 0.0 && s * s <= w.th2 * d2) return kFar;
+  if (al && bl) return kNear;
+  if (bl || (!al && A.w >= B.w)) return kSplitA;
+  return kSplitB;
+}
+
+__device__ inline void put_pair(void* keys, int32_t wide, int32_t shift, int64_t o, uint32_t a, uint32_t b) {
+  if (wide) {
+    uint64_t* k = static_cast<uint64_t*>(keys) + o;
+    k[0] = (uint64_t(a) << shift) | b;
+    k[1] = (uint64_t(b) << shift) | a;
   } else {
-    const double dx = C[3 * a] - C[3 * b], dy = C[3 * a + 1] - C[3 * b + 1], dz = C[3 * a + 2] - C[3 * b + 2];
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    const double s = R[a] + R[b];
-    const bool al = a >= I, bl = b >= I;
-    if (d2 > 0.0 && s * s <= th2 * d2) c = kFar;
-    else if (al && bl) c = kNear;
-    else if (bl || (!al && R[a] >= R[b])) c = kSplitA;
-    else c = kSplitB;
+    uint32_t* k = static_cast<uint32_t*>(keys) + o;
+    k[0] = (a << shift) | b;
+    k[1] = (b << shift) | a;
   }
-  code[t] = c;
-  counts3[t] = c == kSelf ? 3 : (c == kSplitA || c == kSplitB) ? 2 : 0;
-  counts3[n_in + t] = c == kFar ? 2 : 0;
-  counts3[2 * n_in + t] = c == kNear ? 2 : 0;
 }
 
-__global__ void __launch_bounds__(256) walk_emit_kernel(const int2* __restrict__ in, int64_t n_in, int32_t I,
-                                                        const int32_t* __restrict__ left,
-                                                        const int32_t* __restrict__ right,
-                                                        const uint8_t* __restrict__ code,
-                                                        const int32_t* __restrict__ offsets3, int64_t far_base,
-                                                        int64_t near_base, int2* __restrict__ items_out,
-                                                        uint64_t* __restrict__ far, uint64_t* __restrict__ near) {
-  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= n_in) return;
-  const int32_t a = in[t].x, b = in[t].y;
-  const uint8_t c = code[t];
-  const int64_t oi = offsets3[t];
-  switch (c) {
-    case kSelf: {
-      const int32_t la = left[a], ra = right[a];
-      items_out[oi] = make_int2(la, ra);
-      items_out[oi + 1] = make_int2(ra, ra);
-      items_out[oi + 2] = make_int2(la, la);
-      break;
+// One tile of THREADS * rounds frontier items (rounds <= MAXR): every thread
+// classifies its items, the counts of every (round, wave) are scanned in LDS,
+// `reserve(items, far, near)` returns where the tile's outputs start (or -1 where
+// a list is full) and the items are written there, neighbouring lanes next to
+// each other.
+template <int THREADS, int MAXR, typename Reserve>
+__device__ inline void walk_tile(const Walk& w, const int2* __restrict__ in, int64_t n, int64_t base, int rounds,
+                                 int2* __restrict__ out, Reserve reserve) {
+  constexpr int WAVES = THREADS / 64;
+  constexpr int CELLS = MAXR * WAVES;
+  static_assert(CELLS <= 64, "one wave scans the cells");
+  __shared__ int32_t cell[3][64];
+  __shared__ int64_t start[3];
+  const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
+  const uint64_t below = (uint64_t(1) << lane) - 1;
+  uint64_t codes = 0;
+  if (tid < 64)
+    for (int c = 0; c < 3; ++c) cell[c][tid] = 0;
+  __syncthreads();
+#pragma unroll 4
+  for (int r = 0; r < rounds; ++r) {
+    const int64_t t = base + int64_t(r) * THREADS + tid;
+    const uint32_t c = t < n ? walk_code(w, in[t]) : uint32_t(kNone);
+    codes |= uint64_t(c) << (4 * r);
+    const uint64_t self = __ballot(c == kSelf), split = __ballot(c >= kSplitA);
+    const uint64_t fr = __ballot(c == kFar), nr = __ballot(c == kNear);
+    if (lane == 0) {
+      cell[0][r * WAVES + wv] = 3 * __popcll(self) + 2 * __popcll(split);
+      cell[1][r * WAVES + wv] = 2 * __popcll(fr);
+      cell[2][r * WAVES + wv] = 2 * __popcll(nr);
     }
-    case kFar: {
-      const int64_t o = far_base + offsets3[n_in + t];
-      far[o] = (uint64_t(uint32_t(a)) << 32) | uint32_t(b);
-      far[o + 1] = (uint64_t(uint32_t(b)) << 32) | uint32_t(a);
-      break;
+  }
+  __syncthreads();
+  if (wv == 0) {
+    int32_t total[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int32_t own = cell[c][lane];
+      int32_t v = own;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+      }
+      cell[c][lane] = v - own;
+      total[c] = __shfl(v, 63);
     }
-    case kNear: {
-      const int64_t o = near_base + offsets3[2 * n_in + t];
-      const uint32_t ta = uint32_t(a - I), tb = uint32_t(b - I);
-      near[o] = (uint64_t(ta) << 32) | tb;
-      near[o + 1] = (uint64_t(tb) << 32) | ta;
-      break;
+    if (lane < 3) start[lane] = reserve(lane, lane == 0 ? total[0] : lane == 1 ? total[1] : total[2]);
+  }
+  __syncthreads();
+  const int64_t s0 = start[0], s1 = start[1], s2 = start[2];
+  for (int r = 0; r < rounds; ++r) {
+    const uint32_t c = uint32_t(codes >> (4 * r)) & 15u;
+    const uint64_t self = __ballot(c == kSelf), split = __ballot(c >= kSplitA);
+    const uint64_t fr = __ballot(c == kFar), nr = __ballot(c == kNear);
+    if (c == kNone) continue;
+    const int2 it = in[base + int64_t(r) * THREADS + tid];
+    if (c == kFar) {
+      if (s1 >= 0)
+        put_pair(w.far, w.far_wide, w.far_shift, s1 + cell[1][r * WAVES + wv] + 2 * __popcll(fr & below),
+                 uint32_t(it.x), uint32_t(it.y));
+    } else if (c == kNear) {
+      if (s2 >= 0)
+        put_pair(w.near, w.near_wide, w.near_shift, s2 + cell[2][r * WAVES + wv] + 2 * __popcll(nr & below),
+                 uint32_t(it.x - w.I), uint32_t(it.y - w.I));
+    } else if (s0 >= 0) {
+      int2* o = out + s0 + cell[0][r * WAVES + wv] + 3 * __popcll(self & below) + 2 * __popcll(split & below);
+      if (c == kSelf) {
+        const int32_t la = w.left[it.x], ra = w.right[it.x];
+        o[0] = make_int2(la, ra);
+        o[1] = make_int2(ra, ra);
+        o[2] = make_int2(la, la);
+      } else if (c == kSplitA) {
+        o[0] = make_int2(w.right[it.x], it.y);
+        o[1] = make_int2(w.left[it.x], it.y);
+      } else {
+        o[0] = make_int2(it.x, w.right[it.y]);
+        o[1] = make_int2(it.x, w.left[it.y]);
+      }
     }
-    case kSplitA:
-      items_out[oi] = make_int2(right[a], b);
-      items_out[oi + 1] = make_int2(left[a], b);
-      break;
-    case kSplitB:
-      items_out[oi] = make_int2(a, right[b]);
-      items_out[oi + 1] = make_int2(a, left[b]);
-      break;
-    default:
-      break;
+  }
+  __syncthreads();  // cell and start are reused by the next tile
+}
+
+// One breadth-first step over a fixed grid.  Tiles grow with the frontier (up
+// to 4096 items), since each adds to the three shared counters once.
+constexpr int kWalkThreads = 256;
+constexpr int kWalkRounds = 16;
+constexpr int kWalkBlocks = 1024;
+
+__global__ void __launch_bounds__(kWalkThreads) walk_step_kernel(Walk w, int32_t step) {
+  unsigned long long* now = w.st + kSteps + 2 * step;
+  const int64_t n = static_cast<int64_t>(now[0]);
+  const int buf = static_cast<int>(now[1]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) now[3] = n > 0 ? 1 - buf : buf;
+  if (n == 0 || w.st[kOverflow] & kFullFrontier) return;  // unwritten frontier entries are never read
+  const int64_t most = int64_t(gridDim.x) * kWalkThreads;
+  const int rounds = static_cast<int>(min(int64_t(kWalkRounds), (n + most - 1) / most));
+  const int64_t tile = int64_t(rounds) * kWalkThreads;
+  for (int64_t base = blockIdx.x * tile; base < n; base += gridDim.x * tile)
+    walk_tile<kWalkThreads, kWalkRounds>(
+        w, w.frontier[buf], n, base, rounds, w.frontier[1 - buf], [&](int list, int32_t count) -> int64_t {
+          if (count == 0) return 0;
+          unsigned long long* ctr = list == 0 ? now + 2 : list == 1 ? w.st + kFarCount : w.st + kNearCount;
+          const int64_t at = static_cast<int64_t>(atomicAdd(ctr, static_cast<unsigned long long>(count)));
+          const int64_t cap = list == 0 ? w.frontier_cap : list == 1 ? w.far_cap : w.near_cap;
+          if (at + count <= cap) return at;
+          atomicOr(w.st + kOverflow, static_cast<unsigned long long>(list == 0 ? kFullFrontier : list == 1 ? kFullFar : kFullNear));
+          if (list == 0) atomicMax(w.st + kFrontierNeed, static_cast<unsigned long long>(at + count));
+          return -1;
+        });
+}
+
+// Steps of small frontiers (the first and last of a walk, all of a small tree's)
+// in one workgroup until the frontier is empty or outgrows kWalkSmall items.
+constexpr int kWalkSmallThreads = 1024;
+constexpr int kWalkSmall = 2 * kWalkSmallThreads;
+
+__global__ void __launch_bounds__(kWalkSmallThreads) walk_small_kernel(Walk w, int32_t step) {
+  __shared__ int64_t next[3];  // items of the next frontier, far and near entries so far
+  unsigned long long* now = w.st + kSteps + 2 * step;
+  int64_t n = static_cast<int64_t>(now[0]);
+  int buf = static_cast<int>(now[1]);
+  bool full = (w.st[kOverflow] & kFullFrontier) != 0;
+  if (threadIdx.x == 0) {
+    next[1] = static_cast<int64_t>(w.st[kFarCount]);
+    next[2] = static_cast<int64_t>(w.st[kNearCount]);
+  }
+  // n items with n <= kWalkSmall make at most 3 n, and a walk is finite: every
+  // step replaces an item by items of strictly smaller nodes
+  while (n > 0 && n <= kWalkSmall && !full) {
+    if (threadIdx.x == 0) next[0] = 0;
+    const int rounds = n > kWalkSmallThreads ? 2 : 1;
+    walk_tile<kWalkSmallThreads, 2>(w, w.frontier[buf], n, 0, rounds, w.frontier[1 - buf],
+                                    [&](int list, int32_t count) -> int64_t {
+                                      const int64_t at = next[list];
+                                      next[list] = at + count;
+                                      const int64_t cap = list == 0 ? w.frontier_cap : list == 1 ? w.far_cap : w.near_cap;
+                                      if (at + count <= cap) return at;
+                                      atomicOr(w.st + kOverflow, static_cast<unsigned long long>(
+                                                                    list == 0 ? kFullFrontier : list == 1 ? kFullFar : kFullNear));
+                                      if (list == 0) atomicMax(w.st + kFrontierNeed, static_cast<unsigned long long>(at + count));
+                                      return -1;
+                                    });
+    n = next[0];
+    full = n > w.frontier_cap;
+    buf = 1 - buf;
+    __syncthreads();  // everyone has read next[0]
+  }
+  if (threadIdx.x == 0) {
+    w.st[kFarCount] = static_cast<unsigned long long>(next[1]);
+    w.st[kNearCount] = static_cast<unsigned long long>(next[2]);
+    now[2] = static_cast<unsigned long long>(n);
+    now[3] = static_cast<unsigned long long>(buf);
   }
 }
 
@@ -468,6 +633,28 @@ __global__ void __launch_bounds__(256) low_words_kernel(const uint64_t* __restri
                                                         int32_t* __restrict__ col) {
   const int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (k < K) col[k] = static_cast<int32_t>(keys[k] & 0xFFFFFFFFull);
+}
+
+// the same from keys (row << shift) | col of either width
+template <typename K>
+__global__ void __launch_bounds__(256) packed_offsets_kernel(const K* __restrict__ keys, int64_t n, int32_t shift,
+                                                             int32_t rows, int32_t* __restrict__ off) {
+  const int32_t r = blockIdx.x * 256 + threadIdx.x;
+  if (r > rows) return;
+  int64_t lo = 0, hi = n;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (static_cast<int64_t>(keys[mid] >> shift) < r) lo = mid + 1;
+    else hi = mid;
+  }
+  off[r] = static_cast<int32_t>(lo);
+}
+
+template <typename K>
+__global__ void __launch_bounds__(256) packed_cols_kernel(const K* __restrict__ keys, int64_t n, K mask,
+                                                          int32_t* __restrict__ col) {
+  const int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (k < n) col[k] = static_cast<int32_t>(keys[k] & mask);
 }
 
 inline unsigned grid_for(int64_t n, int per_block = 256) {
@@ -617,43 +804,136 @@ int32_t jfm_tree_geometry_pass(void* stream, const int32_t* lev_off_host, int32_
   return jfm::check_launch("jfm_tree_geometry_pass");
 }
 
+int64_t jfm_tree_radius_work(int32_t nodes, int64_t n, int32_t max_depth) {
+  if (nodes < 1 || n < 1 || max_depth < 0) return -1;
+  // nodes of one depth are disjoint: at most n / kSmallRadius large ones, whose
+  // chunks are at most n / kRadiusChunk full ones and one more each
+  return (n / jfm::kRadiusChunk + n / jfm::kSmallRadius + 1) * (int64_t(max_depth) + 1);
+}
+
 int32_t jfm_tree_radius(void* stream, int32_t nodes, int64_t n, const double* pos, const int32_t* perm,
-                        const int32_t* node_range, const double* center, double* scratch, double* radius) {
-  if (nodes < 1 || n < 1 || !pos || !perm || !node_range || !center || !scratch || !radius)
+                        const int32_t* node_range, const double* center, double* scratch, int32_t* work,
+                        int64_t work_cap, double* radius) {
+  if (nodes < 1 || n < 1 || !pos || !perm || !node_range || !center || !scratch || !work || work_cap < 1 ||
+      work_cap > INT32_MAX / 2 || !radius)
     return fail(JFM_ERR_ARG, "jfm_tree_radius: bad argument");
   hipStream_t s = jfm::as_stream(stream);
   jfm::Particles P{pos, nullptr, perm};
-  hipLaunchKernelGGL(jfm::sorted_positions_kernel, dim3(jfm::grid_for(n)), dim3(256), 0, s, P, n, scratch);
+  int2* list = reinterpret_cast<int2*>(work + 2);
+  const int32_t cap = static_cast<int32_t>(work_cap);
+  hipLaunchKernelGGL(jfm::sorted_positions_kernel, dim3(jfm::grid_for(n)), dim3(256), 0, s, P, n, scratch, work);
   hipLaunchKernelGGL(jfm::radius_small_kernel, dim3(jfm::grid_for(nodes, 4)), dim3(256), 0, s, scratch, nodes,
-                     node_range, center, radius);
-  hipLaunchKernelGGL(jfm::radius_big_kernel, dim3(nodes), dim3(1024), 0, s, scratch, nodes, node_range, center,
-                     radius);
+                     node_range, center, radius, list, cap, work);
+  if (n > jfm::kSmallRadius) {
+    hipLaunchKernelGGL(jfm::radius_big_kernel, dim3(jfm::kRadiusBlocks), dim3(256), 0, s, scratch, node_range, center,
+                       list, cap, work, radius);
+    hipLaunchKernelGGL(jfm::radius_root_kernel, dim3(jfm::grid_for(nodes)), dim3(256), 0, s, nodes, node_range,
+                       radius);
+  }
   return jfm::check_launch("jfm_tree_radius");
 }
 
-int32_t jfm_tree_walk_classify(void* stream, int32_t I, const int32_t* items_in, int64_t n_in, const double* center,
-                               const double* radius, double theta, uint8_t* codes, int32_t* counts3) {
-  if (n_in < 0 || n_in > INT32_MAX || I < 0 || !center || !radius || !(theta > 0.0) ||
-      (n_in > 0 && (!items_in || !codes || !counts3)))
-    return fail(JFM_ERR_ARG, "jfm_tree_walk_classify: bad argument");
-  if (n_in == 0) return JFM_OK;
-  hipLaunchKernelGGL(jfm::walk_classify_kernel, dim3(jfm::grid_for(n_in)), dim3(256), 0, jfm::as_stream(stream),
-                     reinterpret_cast<const int2*>(items_in), n_in, I, center, radius, theta * theta, codes, counts3);
-  return jfm::check_launch("jfm_tree_walk_classify");
+int32_t jfm_tree_walk_state_words(int32_t steps) { return steps < 0 ? -1 : jfm::kSteps + 2 * (steps + 1); }
+
+int32_t jfm_tree_pack_nodes(void* stream, int32_t nodes, const double* center, const double* radius, void* node4) {
+  if (nodes < 1 || !center || !radius || !node4) return fail(JFM_ERR_ARG, "jfm_tree_pack_nodes: bad argument");
+  hipLaunchKernelGGL(jfm::pack_nodes_kernel, dim3(jfm::grid_for(nodes)), dim3(256), 0, jfm::as_stream(stream), nodes,
+                     center, radius, static_cast<double4*>(node4));
+  return jfm::check_launch("jfm_tree_pack_nodes");
 }
 
-int32_t jfm_tree_walk_emit(void* stream, int32_t I, const int32_t* items_in, int64_t n_in, const int32_t* left,
-                           const int32_t* right, const uint8_t* codes, const int32_t* offsets3, int64_t far_base,
-                           int64_t near_base, int32_t* items_out, uint64_t* far_keys, uint64_t* near_keys) {
-  if (n_in < 0 || n_in > INT32_MAX || I < 0 || far_base < 0 || near_base < 0 ||
-      (n_in > 0 && (!items_in || !codes || !offsets3 || !items_out || !far_keys || !near_keys)) ||
-      (I > 0 && (!left || !right)))
-    return fail(JFM_ERR_ARG, "jfm_tree_walk_emit: bad argument");
-  if (n_in == 0) return JFM_OK;
-  hipLaunchKernelGGL(jfm::walk_emit_kernel, dim3(jfm::grid_for(n_in)), dim3(256), 0, jfm::as_stream(stream),
-                     reinterpret_cast<const int2*>(items_in), n_in, I, left, right, codes, offsets3, far_base,
-                     near_base, reinterpret_cast<int2*>(items_out), far_keys, near_keys);
-  return jfm::check_launch("jfm_tree_walk_emit");
+int32_t jfm_tree_walk(void* stream, int32_t I, const void* node4, const int32_t* left, const int32_t* right,
+                      double theta, void* frontier0, void* frontier1, int64_t frontier_cap, void* far,
+                      int64_t far_cap, int32_t far_shift, int32_t far_wide, void* near, int64_t near_cap,
+                      int32_t near_shift, int32_t near_wide, uint64_t* state, int32_t first_step, int32_t groups,
+                      int32_t steps_per_group) {
+  if (I < 0 || !node4 || (I > 0 && (!left || !right)) || !(theta > 0.0) || !frontier0 || !frontier1 ||
+      frontier_cap < 1 || !far || far_cap < 0 || !near || near_cap < 0 || !state || first_step < 0 || groups < 1 ||
+      steps_per_group < 0)
+    return fail(JFM_ERR_ARG, "jfm_tree_walk: bad argument");
+  if (far_shift < 1 || far_shift > 31 || near_shift < 1 || near_shift > 31 || (!far_wide && far_shift > 16) ||
+      (!near_wide && near_shift > 16))
+    return fail(JFM_ERR_ARG, "jfm_tree_walk: key shifts out of range");
+  hipStream_t s = jfm::as_stream(stream);
+  jfm::Walk w;
+  w.I = I;
+  w.th2 = theta * theta;
+  w.node = static_cast<const double4*>(node4);
+  w.left = left;
+  w.right = right;
+  w.frontier[0] = static_cast<int2*>(frontier0);
+  w.frontier[1] = static_cast<int2*>(frontier1);
+  w.frontier_cap = frontier_cap;
+  w.far = far;
+  w.far_cap = far_cap;
+  w.far_shift = far_shift;
+  w.far_wide = far_wide;
+  w.near = near;
+  w.near_cap = near_cap;
+  w.near_shift = near_shift;
+  w.near_wide = near_wide;
+  w.st = reinterpret_cast<unsigned long long*>(state);
+  int32_t step = first_step;
+  for (int32_t g = 0; g < groups; ++g) {
+    hipLaunchKernelGGL(jfm::walk_small_kernel, dim3(1), dim3(jfm::kWalkSmallThreads), 0, s, w, step++);
+    for (int32_t k = 0; k < steps_per_group; ++k)
+      hipLaunchKernelGGL(jfm::walk_step_kernel, dim3(jfm::kWalkBlocks), dim3(jfm::kWalkThreads), 0, s, w, step++);
+  }
+  hipLaunchKernelGGL(jfm::walk_small_kernel, dim3(1), dim3(jfm::kWalkSmallThreads), 0, s, w, step);
+  return jfm::check_launch("jfm_tree_walk");
+}
+
+int32_t jfm_sort_packed_scratch_bytes(int64_t n, int32_t wide, int64_t* bytes) {
+  if (!bytes || n < 0 || n > INT32_MAX) return fail(JFM_ERR_ARG, "jfm_sort_packed_scratch_bytes: bad argument");
+  size_t b = 0;
+  hipError_t e;
+  if (wide)
+    e = hipcub::DeviceRadixSort::SortKeys(nullptr, b, static_cast<const uint64_t*>(nullptr),
+                                          static_cast<uint64_t*>(nullptr), static_cast<int>(n), 0, 64);
+  else
+    e = hipcub::DeviceRadixSort::SortKeys(nullptr, b, static_cast<const uint32_t*>(nullptr),
+                                          static_cast<uint32_t*>(nullptr), static_cast<int>(n), 0, 32);
+  if (e != hipSuccess)
+    return fail(JFM_ERR_HIP, std::string("jfm_sort_packed_scratch_bytes: ") + hipGetErrorString(e));
+  *bytes = static_cast<int64_t>(b);
+  return JFM_OK;
+}
+
+int32_t jfm_packed_to_csr(void* stream, int64_t n, int32_t wide, int32_t shift, const void* keys, void* sorted,
+                          void* scratch, int64_t scratch_bytes, int32_t rows, int32_t* off, int32_t* col) {
+  if (n < 0 || n > INT32_MAX || rows < 0 || shift < 1 || shift > 31 || (!wide && shift > 16) || !off ||
+      (n > 0 && (!keys || !sorted || !col)))
+    return fail(JFM_ERR_ARG, "jfm_packed_to_csr: bad argument");
+  hipStream_t s = jfm::as_stream(stream);
+  if (n > 0) {
+    int64_t need = 0;
+    if (int32_t rc = jfm_sort_packed_scratch_bytes(n, wide, &need)) return rc;
+    if (!scratch || scratch_bytes < need) return fail(JFM_ERR_ARG, "jfm_packed_to_csr: scratch too small");
+    size_t b = static_cast<size_t>(scratch_bytes);
+    hipError_t e;
+    if (wide)
+      e = hipcub::DeviceRadixSort::SortKeys(scratch, b, static_cast<const uint64_t*>(keys),
+                                            static_cast<uint64_t*>(sorted), static_cast<int>(n), 0, 2 * shift, s);
+    else
+      e = hipcub::DeviceRadixSort::SortKeys(scratch, b, static_cast<const uint32_t*>(keys),
+                                            static_cast<uint32_t*>(sorted), static_cast<int>(n), 0, 2 * shift, s);
+    if (e != hipSuccess) return fail(JFM_ERR_HIP, std::string("jfm_packed_to_csr: ") + hipGetErrorString(e));
+  }
+  const dim3 ro(jfm::grid_for(int64_t(rows) + 1)), co(jfm::grid_for(n > 0 ? n : 1));
+  if (wide) {
+    hipLaunchKernelGGL(jfm::packed_offsets_kernel<uint64_t>, ro, dim3(256), 0, s, static_cast<const uint64_t*>(sorted),
+                       n, shift, rows, off);
+    if (n > 0)
+      hipLaunchKernelGGL(jfm::packed_cols_kernel<uint64_t>, co, dim3(256), 0, s, static_cast<const uint64_t*>(sorted),
+                         n, (uint64_t(1) << shift) - 1, col);
+  } else {
+    hipLaunchKernelGGL(jfm::packed_offsets_kernel<uint32_t>, ro, dim3(256), 0, s, static_cast<const uint32_t*>(sorted),
+                       n, shift, rows, off);
+    if (n > 0)
+      hipLaunchKernelGGL(jfm::packed_cols_kernel<uint32_t>, co, dim3(256), 0, s, static_cast<const uint32_t*>(sorted),
+                         n, (uint32_t(1) << shift) - 1, col);
+  }
+  return jfm::check_launch("jfm_packed_to_csr");
 }
 
 int32_t jfm_scan_scratch_bytes(int64_t n, int64_t* bytes) {
