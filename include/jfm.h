@@ -212,6 +212,19 @@ int32_t jfm_nonempty_rows(void* stream, int32_t rows, const int32_t* off, uint64
 int32_t jfm_flat_spans(void* stream, int64_t K, const int32_t* pair_tgt, int32_t* span_tgt, int32_t* span_w0,
                        int32_t* span_w1, uint64_t* count);
 
+/* P2P work items of the near CSR near_off [L+1]: leaf l's (1 + its entries) *
+ * leaf_size slots in chunks of chunk_slots (a multiple of leaf_size).
+ * jfm_item_counts: counts3 [3][L] = items, partial rows (items of leaves cut in
+ * several), 1 for such a leaf; jfm_scan_i32 on each row gives offsets3;
+ * jfm_item_emit writes the item and split lists (jfm_p2p_items) up to their
+ * capacities and the three totals. */
+int32_t jfm_item_counts(void* stream, int32_t L, int32_t leaf_size, int32_t chunk_slots, const int32_t* near_off,
+                        int32_t* counts3);
+int32_t jfm_item_emit(void* stream, int32_t L, int32_t leaf_size, int32_t chunk_slots, const int32_t* near_off,
+                      const int32_t* counts3, const int32_t* offsets3, int32_t item_cap, int32_t* leaf, int32_t* s0,
+                      int32_t* s1, int32_t* part, int32_t split_cap, int32_t* split_leaf, int32_t* split_p0,
+                      int32_t* split_p1, int32_t* totals3);
+
 /* Dehnen real multipole swap matrices B_U for degrees 0..p, float64, packed
  * row-major block after block (sum (2l+1)^2 entries); the constants every
  * rotation kernel is compiled with (jaccpot/operators/real_dehnen_q.py:343-470). */

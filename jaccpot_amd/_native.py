@@ -66,6 +66,9 @@ _SIGNATURES = {
     "jfm_sort_packed_scratch_bytes": (c_int32, [c_int64, c_int32, POINTER(c_int64)]),
     "jfm_packed_to_csr": (c_int32, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                     c_void_p, c_void_p]),
+    "jfm_item_counts": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
+    "jfm_item_emit": (c_int32, [c_void_p, c_int32, c_int32, c_int32] + [c_void_p] * 3 + [c_int32] + [c_void_p] * 4
+                      + [c_int32] + [c_void_p] * 4),
     "jfm_scan_scratch_bytes": (c_int32, [c_int64, POINTER(c_int64)]),
     "jfm_scan_i32": (c_int32, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64]),
     "jfm_keys_to_csr": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
@@ -223,7 +226,8 @@ def call(name: str, *args) -> int:
     rc = getattr(load(), name)(*args)
     if name not in ("jfm_direct_scratch_doubles", "jfm_coeff_stride", "jfm_order_supported", "jfm_abi_version",
                     "jfm_mlp_num_params", "jfm_mlp_backward_scratch_floats", "jfm_tree_bounds_scratch_doubles",
-                    "jfm_key_bits", "jfm_tree_radius_work", "jfm_tree_walk_state_words", "jfm_m2l_engine", "jfm_direct_sum_f64_static_max_targets"):
+                    "jfm_key_bits", "jfm_tree_radius_work", "jfm_tree_walk_state_words", "jfm_m2l_engine",
+                    "jfm_direct_sum_f64_static_max_targets"):
         check(rc, name)
     return rc
 

@@ -190,8 +190,8 @@ def fmm_vjp(fmm, state, positions: torch.Tensor, masses: torch.Tensor, acc_bar: 
              state.centers4.data_ptr())
     mbar = torch.zeros_like(state.multipoles)
     cbar4 = torch.zeros((topo.num_nodes, 4), dtype=dt, device=dev)
-    if topo.m2l_targets.size:
-        nt = int(topo.m2l_targets.size)
+    if topo.num_m2l_targets:
+        nt = topo.num_m2l_targets
         if ag is None:
             nat.call("jfm_m2l", s, code, state.order, state.m2l_targets.data_ptr(), nt, state.far_off.data_ptr(),
                      state.far_src.data_ptr(), lbar.data_ptr(), state.centers4.data_ptr(), mbar.data_ptr())

@@ -13,6 +13,8 @@
 //   non-empty rows       targets that have pairs (appended, then sorted)
 //   flat spans           targets whose pairs cross a 64-pair block boundary,
 //                        one per such target, found at its first crossing
+//   P2P items            near lists cut into work items (nearsplit): counts per
+//                        leaf, exclusive scans, one thread per leaf writes
 
 #include <hip/hip_runtime.h>
 
@@ -101,6 +103,53 @@ __global__ void __launch_bounds__(256) flat_spans_kernel(int64_t K, const int32_
 
 inline unsigned grid_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
+// counts [3][L]: items of leaf l, partial rows (items of a split leaf), split leaves
+__global__ void __launch_bounds__(256) item_counts_kernel(int32_t L, int32_t leaf_size, int64_t chunk,
+                                                          const int32_t* __restrict__ near_off,
+                                                          int32_t* __restrict__ counts) {
+  const int32_t l = blockIdx.x * 256 + threadIdx.x;
+  if (l >= L) return;
+  const int64_t slots = (int64_t(near_off[l + 1]) - near_off[l] + 1) * leaf_size;
+  const int32_t c = static_cast<int32_t>((slots + chunk - 1) / chunk);
+  counts[l] = c;
+  counts[L + l] = c > 1 ? c : 0;
+  counts[2 * L + l] = c > 1 ? 1 : 0;
+}
+
+struct ItemLists {
+  int32_t *leaf, *s0, *s1, *part;  // item_cap entries
+  int32_t *split_leaf, *split_p0, *split_p1;  // split_cap entries
+  int32_t item_cap, split_cap;
+};
+
+__global__ void __launch_bounds__(256) item_emit_kernel(int32_t L, int32_t leaf_size, int32_t chunk,
+                                                        const int32_t* __restrict__ near_off,
+                                                        const int32_t* __restrict__ counts,
+                                                        const int32_t* __restrict__ offsets, ItemLists out,
+                                                        int32_t* __restrict__ totals) {
+  const int32_t l = blockIdx.x * 256 + threadIdx.x;
+  if (l >= L) return;
+  const int64_t slots = (int64_t(near_off[l + 1]) - near_off[l] + 1) * leaf_size;
+  const int32_t c = counts[l], first = offsets[l], p0 = offsets[L + l], sp = offsets[2 * L + l];
+  for (int32_t k = 0; k < c && first + k < out.item_cap; ++k) {
+    const int64_t a = int64_t(k) * chunk;
+    out.leaf[first + k] = l;
+    out.s0[first + k] = static_cast<int32_t>(a);
+    out.s1[first + k] = static_cast<int32_t>(min(a + chunk, slots));
+    out.part[first + k] = c > 1 ? p0 + k : -1;
+  }
+  if (c > 1 && sp < out.split_cap) {
+    out.split_leaf[sp] = l;
+    out.split_p0[sp] = p0;
+    out.split_p1[sp] = p0 + c;
+  }
+  if (l == L - 1) {
+    totals[0] = first + c;
+    totals[1] = p0 + counts[L + l];
+    totals[2] = sp + counts[2 * L + l];
+  }
+}
+
 }  // namespace
 }  // namespace jfm
 
@@ -161,6 +210,28 @@ int32_t jfm_flat_spans(void* stream, int64_t K, const int32_t* pair_tgt, int32_t
   hipLaunchKernelGGL(jfm::flat_spans_kernel, dim3(jfm::grid_for(boundaries)), dim3(256), 0, jfm::as_stream(stream), K,
                      pair_tgt, span_tgt, span_w0, span_w1, reinterpret_cast<unsigned long long*>(count));
   return jfm::check_launch("jfm_flat_spans");
+}
+
+int32_t jfm_item_counts(void* stream, int32_t L, int32_t leaf_size, int32_t chunk_slots, const int32_t* near_off,
+                        int32_t* counts3) {
+  if (L < 1 || leaf_size < 1 || chunk_slots < 1 || !near_off || !counts3)
+    return fail(JFM_ERR_ARG, "jfm_item_counts: bad argument");
+  jfm::item_counts_kernel<<<(L + 255) / 256, 256, 0, jfm::as_stream(stream)>>>(L, leaf_size, chunk_slots, near_off,
+                                                                              counts3);
+  return jfm::check_launch("jfm_item_counts");
+}
+
+int32_t jfm_item_emit(void* stream, int32_t L, int32_t leaf_size, int32_t chunk_slots, const int32_t* near_off,
+                      const int32_t* counts3, const int32_t* offsets3, int32_t item_cap, int32_t* leaf, int32_t* s0,
+                      int32_t* s1, int32_t* part, int32_t split_cap, int32_t* split_leaf, int32_t* split_p0,
+                      int32_t* split_p1, int32_t* totals3) {
+  if (L < 1 || leaf_size < 1 || chunk_slots < 1 || !near_off || !counts3 || !offsets3 || item_cap < 1 || !leaf ||
+      !s0 || !s1 || !part || split_cap < 1 || !split_leaf || !split_p0 || !split_p1 || !totals3)
+    return fail(JFM_ERR_ARG, "jfm_item_emit: bad argument");
+  const jfm::ItemLists out{leaf, s0, s1, part, split_leaf, split_p0, split_p1, item_cap, split_cap};
+  jfm::item_emit_kernel<<<(L + 255) / 256, 256, 0, jfm::as_stream(stream)>>>(L, leaf_size, chunk_slots, near_off,
+                                                                            counts3, offsets3, out, totals3);
+  return jfm::check_launch("jfm_item_emit");
 }
 
 }  // extern "C"

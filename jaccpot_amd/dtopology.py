@@ -5,10 +5,9 @@ builders for the reference, jaccpot/runtime/fmm_state.py:630-800,
 runtime/_interaction_cache.py:523,564), run as libjfm device kernels
 (``csrc/treebuild.hip``): bounds, Morton codes, stable radix sort, radix tree,
 levels, centres of mass and radii, breadth-first dual-tree walk, CSR lists.
-Returns a ``Topology`` (host arrays, so every host consumer works unchanged;
-the three largest are copied from the device on first read) with the device
-arrays in ``extra["device"]`` so that ``prepare_state`` does not upload them
-again.
+Returns a ``Topology`` (its host arrays are copied from the device when first
+read, so every host consumer works unchanged) with the device arrays in
+``extra["device"]`` so that ``prepare_state`` does not upload them again.
 """
 
 from __future__ import annotations
@@ -26,24 +25,47 @@ MAX_TREE_HEIGHT = 128  # depths of a radix tree over 63-bit codes with index tie
 
 
 class _Lazy:
-    """A device array whose host copy is made on first access."""
+    """A device array whose host copy is made on first access (from whatever
+    stream that happens on, so after a device-wide wait)."""
 
     __slots__ = ("t",)
 
     def __init__(self, t: torch.Tensor):
         self.t = t
 
+    def host(self) -> np.ndarray:
+        torch.cuda.synchronize(self.t.device)
+        return self.t.cpu().numpy()
+
+
+class LazyExtra(dict):
+    """A dict whose ``_Lazy`` values become host arrays when first read by key."""
+
+    def __getitem__(self, key):
+        v = dict.__getitem__(self, key)
+        if type(v) is _Lazy:
+            v = v.host()
+            self[key] = v
+        return v
+
+    def get(self, key, default=None):
+        return self[key] if key in self else default
+
 
 class DeviceTopology(Topology):
-    """``Topology`` whose largest host arrays (perm, far_src, near_src) are copied
-    from the device only when first read; the device build never needs them."""
+    """``Topology`` whose host arrays are copied from the device only when first
+    read; the device build and the evaluation never need them."""
 
     def __getattribute__(self, name):
         v = object.__getattribute__(self, name)
         if type(v) is _Lazy:
-            v = v.t.cpu().numpy()
+            v = v.host()
             object.__setattr__(self, name, v)
         return v
+
+    @property
+    def num_m2l_targets(self) -> int:
+        return int(self.extra["num_m2l_targets"])
 
     @property
     def num_far_pairs(self) -> int:
@@ -152,8 +174,10 @@ def _packed_csr(keys: torch.Tensor, n: int, shift: int, wide: int, rows: int):
 
 
 def build_topology_device(x: torch.Tensor, m: torch.Tensor, *, leaf_size: int, theta: float,
-                          bounds=None) -> Topology:
-    """Build the topology for input-order float64 device tensors x [N,3], m [N]."""
+                          bounds=None, check_masses: bool = False) -> Topology:
+    """Build the topology for input-order float64 device tensors x [N,3], m [N].
+    ``check_masses``: masses that are not finite raise as positions do.  The last
+    kernels (the near list's sort) may still run when this returns."""
     if x.dtype != torch.float64 or m.dtype != torch.float64 or x.device.type != "cuda":
         raise ValueError("build_topology_device needs float64 CUDA tensors")
     if x.ndim != 2 or x.shape[1] != 3 or m.shape != (x.shape[0],):
@@ -184,6 +208,8 @@ def build_topology_device(x: torch.Tensor, m: torch.Tensor, *, leaf_size: int, t
         b6 = torch.empty(6, dtype=torch.float64, device=dev)
     nat.call("jfm_tree_bounds", s, x.data_ptr(), n, 1 if bounds is not None else 0, bscratch.data_ptr(),
              b6.data_ptr(), flags.data_ptr())
+    if check_masses:
+        flags |= (~torch.isfinite(m)).any().to(torch.int32) * 4
     codes = torch.empty(n, dtype=torch.int64, device=dev)
     index = torch.empty(n, dtype=torch.int32, device=dev)
     nat.call("jfm_tree_morton", s, x.data_ptr(), n, b6.data_ptr(), codes.data_ptr(), index.data_ptr())
@@ -211,13 +237,15 @@ def build_topology_device(x: torch.Tensor, m: torch.Tensor, *, leaf_size: int, t
         m2m_off_d, m2m_nodes = _csr(sk, MAX_TREE_HEIGHT + 1)
         sk, _ = _sort_u64(l2l_keys[: nodes - 1], 32 + _key_bits(MAX_TREE_HEIGHT))
         l2l_off_d, l2l_nodes = _csr(sk, MAX_TREE_HEIGHT)
-        hdr = torch.cat([flags, maxd, m2m_off_d, l2l_off_d]).cpu().numpy()
+        shallow = torch.zeros(14, dtype=torch.int32, device=dev)  # nodes of depths 1 to 3, at most
+        shallow[: min(14, nodes - 1)] = l2l_nodes[:14]
+        hdr = torch.cat([flags, maxd, m2m_off_d, l2l_off_d, shallow]).cpu().numpy()
     else:
         m2m_nodes = torch.empty(0, dtype=torch.int32, device=dev)
         l2l_nodes = torch.empty(0, dtype=torch.int32, device=dev)
         hdr = torch.cat([flags, maxd]).cpu().numpy()
-    if hdr[0] & 1:
-        raise ValueError("positions must be finite")
+    if hdr[0] & 5:
+        raise ValueError("positions and masses must be finite" if check_masses else "positions must be finite")
     if hdr[0] & 2:
         raise RuntimeError("device topology build: parent chain exceeds the maximum tree height")
     D = int(hdr[1])
@@ -252,34 +280,29 @@ def build_topology_device(x: torch.Tensor, m: torch.Tensor, *, leaf_size: int, t
     del node4
     far_off, far_src = _packed_csr(fk, n_far, fb, fw, nodes)
     del fk
+    m2l_targets = torch.nonzero(far_off[1:] > far_off[:-1]).reshape(-1).to(torch.int32)
     near_off, near_src = _packed_csr(nk, n_near, nb, nw, L)
     del nk
-    torch.cuda.synchronize(dev)
     device = dict(perm=perm, parent=parent, left=left, right=right, node_range=node_range, depth=depth,
                   center=center, radius=radius, mass=mass, far_off=far_off, far_src=far_src, near_off=near_off,
-                  near_src=near_src, m2m_nodes=m2m_nodes, l2l_nodes=l2l_nodes, sorted_codes=sorted_codes,
-                  bounds=bounds_used)
-    t1 = time.perf_counter()
-
-    def h(t):
-        return t.cpu().numpy()
-
-    far_off_h = h(far_off)
+                  near_src=near_src, m2m_nodes=m2m_nodes, l2l_nodes=l2l_nodes, m2l_targets=m2l_targets,
+                  sorted_codes=sorted_codes, bounds=bounds_used)
     topo = DeviceTopology(
         num_particles=n, leaf_size=int(leaf_size), num_leaves=L, num_internal=I, num_nodes=nodes, max_depth=D,
-        theta=float(theta), perm=_Lazy(perm), parent=h(parent), left=h(left[:I]), right=h(right[:I]),
-        node_range=h(node_range), depth=h(depth), center=h(center), radius=h(radius), mass=h(mass),
-        far_off=far_off_h, far_src=_Lazy(far_src), near_off=h(near_off), near_src=_Lazy(near_src),
-        m2m_nodes=h(m2m_nodes), m2m_off=m2m_off.astype(np.int32), l2l_nodes=h(l2l_nodes),
-        l2l_off=l2l_off.astype(np.int32),
-        m2l_targets=np.nonzero(np.diff(far_off_h) > 0)[0].astype(np.int32),
-        build_seconds=0.0,
+        theta=float(theta), perm=_Lazy(perm), parent=_Lazy(parent), left=_Lazy(left[:I]), right=_Lazy(right[:I]),
+        node_range=_Lazy(node_range), depth=_Lazy(depth), center=_Lazy(center), radius=_Lazy(radius),
+        mass=_Lazy(mass), far_off=_Lazy(far_off), far_src=_Lazy(far_src), near_off=_Lazy(near_off),
+        near_src=_Lazy(near_src), m2m_nodes=_Lazy(m2m_nodes), m2m_off=m2m_off, l2l_nodes=_Lazy(l2l_nodes),
+        l2l_off=l2l_off, m2l_targets=_Lazy(m2l_targets), build_seconds=0.0,
     )
     topo.extra["num_far_pairs"] = n_far
     topo.extra["num_near_entries"] = n_near
+    topo.extra["num_m2l_targets"] = int(m2l_targets.numel())
+    if I > 0:
+        topo.extra["shallow_nodes"] = nat.host_i32(hdr[2 + 2 * MAX_TREE_HEIGHT + 3:])
     topo.build_seconds = time.perf_counter() - t0
     topo.extra["device"] = device
-    topo.extra["device_build_seconds"] = t1 - t0
+    topo.extra["device_build_seconds"] = topo.build_seconds
     return topo
 
 

@@ -52,16 +52,17 @@ def _as_device_i32(a, device) -> torch.Tensor:
     return torch.as_tensor(np.ascontiguousarray(a, np.int32)).to(device)
 
 
-def build_flat_list(tgt, src, gear: int, dtype: torch.dtype, device) -> FlatList:
+def build_flat_list(tgt, src, gear: int, dtype: torch.dtype, device, grouped: bool = False) -> FlatList:
     """``tgt``/``src`` [K] (numpy arrays or device tensors): target and source node
-    of every pair, grouped by target in ascending order.  The spanning targets
-    are found on the device (``jfm_flat_spans``)."""
+    of every pair, grouped by target in ascending order (``grouped``: known to be,
+    not checked).  The spanning targets are found on the device
+    (``jfm_flat_spans``)."""
     pair_tgt = _as_device_i32(tgt, device)
     pair_src = _as_device_i32(src, device)
     K = int(pair_tgt.numel())
     if K != int(pair_src.numel()):
         raise ValueError("tgt and src must have the same length")
-    if K > 1 and bool((pair_tgt[1:] < pair_tgt[:-1]).any()):
+    if not grouped and K > 1 and bool((pair_tgt[1:] < pair_tgt[:-1]).any()):
         raise ValueError("pairs must be grouped by target in ascending order")
     n_scr = int(nat.load().jfm_m2l_flat_scratch_size(int(gear), K))
     if n_scr < 0:

@@ -22,11 +22,14 @@ gear.  The decision and both error figures are recorded in
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import torch
 
 from . import _native as nat
 from .direct import direct_sum_gravitational_acceleration
+from .nearsplit import P2PItems
 
 # relative force errors below this are float32 rounding, not truncation
 NOISE_FLOOR = 2e-6
@@ -35,6 +38,45 @@ NOISE_FLOOR = 2e-6
 def _errors(acc: torch.Tensor, ref: torch.Tensor) -> np.ndarray:
     a = acc.to(torch.float64)
     return (torch.linalg.norm(a - ref, dim=1) / torch.linalg.norm(ref, dim=1).clamp_min(1e-300)).cpu().numpy()
+
+
+def _near_rows(fmm, state, targets: torch.Tensor) -> torch.Tensor:
+    """Near-field accelerations [N, 3] (input order) of the leaves that hold ``targets``."""
+    topo = state.topology
+    dev = state.device
+    n, leaf = topo.num_particles, topo.leaf_size
+    wanted = torch.zeros(n, dtype=torch.bool, device=dev)
+    wanted[targets] = True
+    of_leaf = torch.zeros(topo.num_leaves * leaf, dtype=torch.bool, device=dev)
+    of_leaf[:n] = wanted[state.perm.long()]
+    of_leaf = of_leaf.view(topo.num_leaves, leaf).any(1)
+    items = state.extra.get("p2p_items")
+    if items is None:
+        rows = torch.nonzero(of_leaf).reshape(-1)
+        slots = ((state.near_off[1:] - state.near_off[:-1] + 1) * leaf)[rows]
+        none = torch.zeros(1, dtype=torch.int32, device=dev)
+        some = P2PItems(num_items=int(rows.numel()), leaf=rows.to(torch.int32), s0=torch.zeros_like(slots), s1=slots,
+                        part=torch.full_like(slots, -1), num_part=0,
+                        partials=torch.zeros((1, leaf, 4), dtype=state.dtype, device=dev), num_split=0,
+                        split_leaf=none, split_p0=none, split_p1=none)
+    else:
+        k = torch.nonzero(of_leaf[items.leaf.long()]).reshape(-1)
+        c = torch.nonzero(of_leaf[items.split_leaf.long()]).reshape(-1)
+        some = dataclasses.replace(items, num_items=int(k.numel()), leaf=items.leaf[k], s0=items.s0[k], s1=items.s1[k],
+                                   part=items.part[k], num_split=int(c.numel()), split_leaf=items.split_leaf[c],
+                                   split_p0=items.split_p0[c], split_p1=items.split_p1[c])
+    acc = torch.zeros((n, 3), dtype=state.dtype, device=dev)
+    fmm._p2p_items(state, some, acc, None, nat.EVAL_COMPENSATED if state.compensated else 0, accumulate=False)
+    return acc
+
+
+def _with_far_field(state, acc: torch.Tensor) -> torch.Tensor:
+    """``acc`` (near field, input order) with the far field of the state's locals added."""
+    topo = state.topology
+    nat.call("jfm_l2p", nat.current_stream(), nat.dtype_code(state.dtype), state.order, state.pos4.data_ptr(),
+             topo.num_particles, topo.leaf_size, topo.num_internal, state.locals.data_ptr(),
+             state.centers4.data_ptr(), state.G, state.perm.data_ptr(), acc.data_ptr(), None, 1)
+    return acc
 
 
 def judge_learned_orders(fmm, state, positions: torch.Tensor, masses: torch.Tensor, *, num_targets: int,
@@ -53,8 +95,10 @@ def judge_learned_orders(fmm, state, positions: torch.Tensor, masses: torch.Tens
     ref = direct_sum_gravitational_acceleration(positions, masses, G=state.G, softening=state.softening,
                                                 target_indices=tgt)
 
-    acc = torch.empty((n, 3), dtype=state.dtype, device=state.device)
-    fmm._evaluate_device(state, acc, None)
+    # the near field does not depend on the orders: once, and only for the
+    # leaves that hold targets (rows of other leaves stay unwritten)
+    near = _near_rows(fmm, state, tgt_d)
+    acc = _with_far_field(state, near.clone())
     err_learned = _errors(acc[tgt_d], ref)
     locals_learned = state.locals.clone()
 
@@ -62,8 +106,7 @@ def judge_learned_orders(fmm, state, positions: torch.Tensor, masses: torch.Tens
     state.extra["gears"] = None
     s = nat.current_stream()
     fmm._downward(state, s, nat.dtype_code(state.dtype))
-    fmm._evaluate_device(state, acc, None)
-    err_plain = _errors(acc[tgt_d], ref)
+    err_plain = _errors(_with_far_field(state, near)[tgt_d], ref)
 
     med_l, med_p = float(np.median(err_learned)), float(np.median(err_plain))
     accepted = med_l <= factor * med_p + NOISE_FLOOR

@@ -191,7 +191,8 @@ def pair_features(state) -> torch.Tensor:
     K = topo.num_far_pairs
     tgt, src, rad = pair_arrays(state)
     X = torch.empty((K, NUM_FEATURES), dtype=torch.float32, device=state.device)
-    total = float(topo.mass[0])
+    mass = topo.extra.get("device", {}).get("mass")
+    total = float(topo.mass[0] if mass is None else mass[0])
     nat.call("jfm_pair_features", nat.current_stream(), state.order, K, tgt.data_ptr(), src.data_ptr(),
              state.multipoles.data_ptr(), state.centers4.data_ptr(), rad.data_ptr(), total, X.data_ptr())
     return X
@@ -289,5 +290,5 @@ def build_gear_schedule(state, gear_of_pair, gears: Sequence[int]) -> GearSchedu
         offsets.append(off)
         sources.append(src if n else one)
         num_targets.append(nt)
-        flat.append(build_flat_list(pt, ps, int(gear), state.dtype, dev) if prefers_flat(n, nt) else None)
+        flat.append(build_flat_list(pt, ps, int(gear), state.dtype, dev, grouped=True) if prefers_flat(n, nt) else None)
     return GearSchedule(tuple(int(x) for x in gears), targets, num_targets, offsets, sources, counts, flops, flat)

@@ -244,7 +244,7 @@ def build_mutual_state(topology: MutualTopology, *, softening: float, G: float =
     ``near_chunk_size``, ``pallas_interpret`` and ``index_dtype`` select the
     reference's JAX lanes and change nothing here."""
     from .flatlist import build_flat_list, pair_targets
-    from .nearsplit import build_p2p_items
+    from .nearsplit import near_items
 
     del index_dtype
     prep = topology.prepared
@@ -265,7 +265,9 @@ def build_mutual_state(topology: MutualTopology, *, softening: float, G: float =
         return torch.as_tensor(np.ascontiguousarray(a, np.int32)).to(dev)
 
     K = prep.topology.num_far_pairs
-    flat = build_flat_list(pair_targets(prep), prep.far_src[:K], prep.order, prep.dtype, dev) if K else None
+    flat = None
+    if K:
+        flat = build_flat_list(pair_targets(prep), prep.far_src[:K], prep.order, prep.dtype, dev, grouped=True)
     n = topology.num_particles
     st = MutualFMMState(
         prepared=prep, near_a=d32(topology.near_a - I), near_b=d32(topology.near_b - I),
@@ -275,7 +277,7 @@ def build_mutual_state(topology: MutualTopology, *, softening: float, G: float =
         order=int(topology.order), use_pallas=bool(use_pallas), near_chunk_size=near_chunk_size,
         pallas_interpret=bool(pallas_interpret), num_particles_=n, num_near_pairs=topology.num_near_pairs,
         num_far_pairs=topology.num_far_pairs, flat=flat, level_off=np.asarray(prep.topology.m2m_off),
-        near_items=build_p2p_items(np.asarray(prep.topology.near_off), prep.topology.leaf_size, prep.dtype, dev))
+        near_items=near_items(prep.topology, prep.dtype, dev))
     st.buffers = {
         "far_acc": torch.empty((n, 3), dtype=prep.dtype, device=dev),
         "rung_sorted": torch.empty(n, dtype=torch.int32, device=dev),
@@ -507,9 +509,9 @@ def _vjp(st: MutualFMMState, x: torch.Tensor, m: torch.Tensor, lw, acc_bar: torc
     _tree_level(prep, prep.m2m_nodes, topo.m2m_off, "m2m", lbar, code, s)  # l2l^T
     mbar = torch.zeros_like(prep.multipoles)
     cbar4 = torch.zeros((topo.num_nodes, 4), dtype=dt, device=dev)
-    if topo.m2l_targets.size:
+    if topo.num_m2l_targets:
         _far_m2l(st, lw, lbar, mbar, code, s)  # m2l^T on the symmetric list
-        nt = int(topo.m2l_targets.size)
+        nt = topo.num_m2l_targets
         if lw is not None:
             nat.call("jfm_center_adjoint_weighted", s, code, prep.order, prep.m2l_targets.data_ptr(), nt,
                      prep.far_off.data_ptr(), prep.far_src.data_ptr(), st.buffers["node_rung"].data_ptr(),

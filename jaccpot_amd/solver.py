@@ -27,8 +27,8 @@ import torch
 
 from . import _native as nat
 from .flatlist import build_flat_list, launch_flat, pair_targets, prefers_flat
-from .nearsplit import build_p2p_items
-from .dtopology import build_topology_device
+from .nearsplit import near_items
+from .dtopology import LazyExtra, _Lazy, build_topology_device
 from .topology import Topology, build_topology
 
 _PRESETS = ("fast", "balanced", "accurate", "large_n_gpu")
@@ -79,7 +79,7 @@ class FMMPreparedState:
     multipoles: torch.Tensor
     locals: torch.Tensor
     compensated: bool = True
-    extra: dict = field(default_factory=dict)
+    extra: dict = field(default_factory=LazyExtra)
 
     @property
     def num_particles(self) -> int:
@@ -262,22 +262,24 @@ class FastMultipoleMethod:
 
     # ------------------------------------------------------------------ utils
     def _as_inputs(self, positions, masses):
+        """Float64 device tensors of the inputs and what the outputs are to look like."""
         if isinstance(positions, torch.Tensor):
             kind, in_dtype, in_dev = "torch", positions.dtype, positions.device
-            x_host = positions.detach().to("cpu", torch.float64).numpy()
-            m_host = torch.as_tensor(masses).detach().to("cpu", torch.float64).numpy()
+            x = positions.detach()
+            m = torch.as_tensor(masses).detach()
         else:
             x_np = np.asarray(positions)
             kind, in_dtype, in_dev = "numpy", x_np.dtype, None
-            x_host = np.asarray(x_np, np.float64)
-            m_host = np.asarray(masses, np.float64)
-        if x_host.ndim != 2 or x_host.shape[1] != 3:
+            # float32 arrays are widened on the GPU
+            x = torch.as_tensor(np.asarray(x_np, x_np.dtype if x_np.dtype == np.float32 else np.float64))
+            m = torch.as_tensor(np.asarray(masses, np.float64))
+        if x.ndim != 2 or x.shape[1] != 3:
             raise ValueError("positions must have shape (N, 3)")
-        if m_host.shape != (x_host.shape[0],):
+        if m.shape != (x.shape[0],):
             raise ValueError("masses must have shape (N,) matching positions")
-        if x_host.shape[0] < 1:
+        if x.shape[0] < 1:
             raise ValueError("need at least one particle")
-        return x_host, m_host, kind, in_dtype, in_dev
+        return x.to(self.device, torch.float64), m.to(self.device, torch.float64), kind, in_dtype, in_dev
 
     def _work_dtype(self, in_dtype) -> torch.dtype:
         if self.working_dtype is not None:
@@ -314,22 +316,21 @@ class FastMultipoleMethod:
         th = self.theta if theta is None else float(theta)
         if not (th > 0.0):
             raise ValueError("theta must be > 0")
-        x_host, m_host, kind, in_dtype, in_dev = self._as_inputs(positions, masses)
-        if not np.all(np.isfinite(x_host)) or not np.all(np.isfinite(m_host)):
-            raise ValueError("positions and masses must be finite")
+        xd, md, kind, in_dtype, in_dev = self._as_inputs(positions, masses)
+        # the device build finds values that are not finite itself
+        if self.tree_build != "device" or self.reuse_topology:
+            if not bool((torch.isfinite(xd).all() & torch.isfinite(md).all()).item()):
+                raise ValueError("positions and masses must be finite")
         dtype = self._work_dtype(in_dtype)
-        dev = self.device
-        xd = torch.as_tensor(x_host, device=dev)
-        md = torch.as_tensor(m_host, device=dev)
-        key = (x_host.shape[0], int(leaf_size), p, th, dtype, None if bounds is None else
+        key = (int(xd.shape[0]), int(leaf_size), p, th, dtype, None if bounds is None else
                tuple(np.concatenate([np.asarray(bounds[0], float), np.asarray(bounds[1], float)]).tolist()))
         reused = self._try_reuse(key, xd, md, bounds, kind, in_dtype, in_dev)
         if reused is not None:
             return reused
         if self.tree_build == "device":
-            topo = build_topology_device(xd, md, leaf_size=int(leaf_size), theta=th, bounds=bounds)
+            topo = build_topology_device(xd, md, leaf_size=int(leaf_size), theta=th, bounds=bounds, check_masses=True)
         else:
-            topo = build_topology(x_host, m_host, leaf_size=int(leaf_size), theta=th, bounds=bounds,
+            topo = build_topology(xd.cpu().numpy(), md.cpu().numpy(), leaf_size=int(leaf_size), theta=th, bounds=bounds,
                                   num_threads=self.num_threads)
         on_dev = topo.extra.get("device", {})
         state = self._state_from_topology(topo, p, dtype, th, kind, in_dtype, in_dev,
@@ -385,11 +386,11 @@ class FastMultipoleMethod:
         )
         if mixed:
             state.extra["mixed"] = self._mixed_schedule(topo, p, dev)
-        if prefers_flat(topo.num_far_pairs, int(topo.m2l_targets.size)):
+        if prefers_flat(topo.num_far_pairs, topo.num_m2l_targets):
             state.extra["flat"] = build_flat_list(pair_targets(state), state.far_src[: topo.num_far_pairs], p, dtype,
-                                                  dev)
+                                                  dev, grouped=True)
         if split_near:
-            state.extra["p2p_items"] = build_p2p_items(topo.near_off, topo.leaf_size, dtype, dev)
+            state.extra["p2p_items"] = near_items(topo, dtype, dev)
         return state
 
     def save_prepared_state(self, state: FMMPreparedState, path) -> None:
@@ -412,7 +413,7 @@ class FastMultipoleMethod:
         import copy
         import dataclasses
 
-        from .dtopology import DeviceTopology, _Lazy, sorted_morton
+        from .dtopology import DeviceTopology, sorted_morton
 
         r = self._reuse
         if not self.reuse_topology or r is None or r["key"] != key or r["count"] >= self.rebuild_every - 1:
@@ -428,7 +429,8 @@ class FastMultipoleMethod:
         state = dataclasses.replace(
             old, topology=topo, perm=perm, input_kind=kind, input_dtype=in_dtype, input_device=in_dev,
             pos4=torch.empty_like(old.pos4), centers4=torch.zeros_like(old.centers4),
-            multipoles=torch.zeros_like(old.multipoles), locals=torch.zeros_like(old.locals), extra=dict(old.extra))
+            multipoles=torch.zeros_like(old.multipoles), locals=torch.zeros_like(old.locals),
+            extra=LazyExtra(old.extra))
         if "mixed" in state.extra:
             state.extra["mixed"] = self._mixed_schedule(topo, state.order, state.device)
         self.refresh_prepared_state(state, xd, md)
@@ -457,7 +459,7 @@ class FastMultipoleMethod:
         X = pair_features(state)
         g = self.order_model.select_gears(X, self.gear_tolerance, state, budget=self.gear_budget)
         state.extra["gears"] = build_gear_schedule(state, g, gears)
-        state.extra["gear_of_pair"] = g.cpu().numpy()
+        state.extra["gear_of_pair"] = _Lazy(g)
 
     def refresh_prepared_state(self, state: FMMPreparedState, positions: torch.Tensor, masses: torch.Tensor) -> None:
         """Re-run gather + upward + downward at the state's frozen topology.
@@ -481,14 +483,19 @@ class FastMultipoleMethod:
     def _mixed_schedule(topo: Topology, p: int, dev) -> dict:
         """Shadow rows and level tables for the float64 top three levels."""
         I = topo.num_internal
-        depth = topo.depth
-        top = np.nonzero(depth[:I] <= 2)[0].astype(np.int32)
-        shadow = np.full(topo.num_nodes, -1, np.int32)
-        shadow[top] = np.arange(top.size, dtype=np.int32)
-        m2m_levels = [top[depth[top] == d] for d in (2, 1, 0)]
+        near_root = topo.extra.get("shallow_nodes")
+        if near_root is None:
+            by_depth = [np.nonzero(topo.depth == d)[0].astype(np.int32) for d in range(4)]
+        else:  # the head of the downward schedule: depths 1, 2 and 3
+            off = topo.l2l_off
+            by_depth = [np.zeros(1, np.int32)] + [near_root[off[d - 1]:off[d]] if d < len(off) else near_root[:0]
+                                                  for d in (1, 2, 3)]
+        m2m_levels = [by_depth[d][by_depth[d] < I] for d in (2, 1, 0)]
+        top = np.sort(np.concatenate(m2m_levels)).astype(np.int32)
+        shadow = torch.full((topo.num_nodes,), -1, dtype=torch.int32, device=dev)
         m2m_nodes = np.concatenate(m2m_levels) if top.size else np.zeros(0, np.int32)
         m2m_off = np.concatenate([[0], np.cumsum([len(v) for v in m2m_levels])]).astype(np.int32)
-        l2l_levels = [np.nonzero(depth == d)[0].astype(np.int32) for d in (1, 2, 3)]
+        l2l_levels = by_depth[1:]
         l2l_nodes = np.concatenate(l2l_levels)
         l2l_off = np.concatenate([[0], np.cumsum([len(v) for v in l2l_levels])]).astype(np.int32)
 
@@ -497,8 +504,11 @@ class FastMultipoleMethod:
 
         cs64 = nat.coeff_stride(p, torch.float64)
         ntop = max(int(top.size), 1)
+        top_d = dev_i32(top)
+        if top.size:
+            shadow[top_d.long()] = torch.arange(top.size, dtype=torch.int32, device=dev)
         return {
-            "top": dev_i32(top), "ntop": int(top.size), "shadow": dev_i32(shadow),
+            "top": top_d, "ntop": int(top.size), "shadow": shadow,
             "m2m_nodes": dev_i32(m2m_nodes), "m2m_off": dev_i32(m2m_off), "m2m_off_host": m2m_off,
             "l2l_nodes": dev_i32(l2l_nodes), "l2l_off": dev_i32(l2l_off), "l2l_off_host": l2l_off,
             "mult64": torch.zeros((ntop, cs64), dtype=torch.float64, device=dev),
@@ -553,8 +563,8 @@ class FastMultipoleMethod:
                              state.multipoles.data_ptr(), state.centers4.data_ptr(), state.locals.data_ptr())
         elif state.extra.get("flat") is not None:
             launch_flat(state.extra["flat"], s, code, state.order, state.multipoles, state.centers4, state.locals)
-        elif topo.m2l_targets.size:
-            nat.call("jfm_m2l", s, code, state.order, state.m2l_targets.data_ptr(), int(topo.m2l_targets.size),
+        elif topo.num_m2l_targets:
+            nat.call("jfm_m2l", s, code, state.order, state.m2l_targets.data_ptr(), topo.num_m2l_targets,
                      state.far_off.data_ptr(), state.far_src.data_ptr(), state.multipoles.data_ptr(),
                      state.centers4.data_ptr(), state.locals.data_ptr())
 

@@ -56,6 +56,10 @@ class Topology:
     def num_near_entries(self) -> int:
         return int(self.near_src.shape[0])
 
+    @property
+    def num_m2l_targets(self) -> int:
+        return int(self.m2l_targets.shape[0])
+
     def p2p_interactions(self) -> int:
         """Pairwise interactions the P2P kernel evaluates (self pairs excluded)."""
         counts = (self.node_range[self.num_internal:, 1] - self.node_range[self.num_internal:, 0] + 1).astype(np.int64)
