@@ -63,6 +63,22 @@ __host__ __device__ __forceinline__ T dev_sqrt(T x) {
   return sqrt(x);
 }
 
+// 1/sqrt(x) for x > 0.  float32: v_rsq_f32 (about 1 ulp); float64: the v_rsq_f64
+// estimate y with one third-order step, y (1 + e/2 + 3e^2/8) with e = 1 - x y^2
+// (the relative error is cubed), 7 instructions against about 35 of a square root
+// and a division.  The minimum turns the NaN of x = inf and x = 0 into e = 1, which
+// leaves y = 0 and y = inf.
+template <typename T>
+__device__ __forceinline__ T fast_rsqrt(T x) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_amdgcn_rsqf(x);
+  } else {
+    const T y = __builtin_amdgcn_rsq(x);
+    const T e = fmin(fma(-(x * y), y, T(1)), T(1));
+    return fma(y * e, fma(e, T(0.375), T(0.5)), y);
+  }
+}
+
 // Per-pair alignment trig: cos/sin of m*az and m*ax for m = 0..P.
 template <typename T, int P>
 struct Align {

@@ -2,19 +2,20 @@
 // leaves of every target leaf, plus the fused evaluate entry point
 // (L2P far field + P2P near field + combine + un-permute).
 //
-// Mapping: one 256-thread workgroup per target leaf.  Thread t owns target
-// t % WT of the leaf (WT = leaf width rounded up to a power of two) and source
-// partition t / WT.  The leaf's source slots (self leaf first, then the near
-// leaves, each leaf_size slots wide) stream through LDS in tiles; inside a
-// tile partition q takes slots q, q + NPART, ... so every lane of a wave reads
-// one broadcast address per interaction and the tail tile stays balanced.
-// The next tile's sources are fetched into registers while the current one is
-// consumed, with the near-list entries loaded one tile further ahead than
-// the positions they address (no load is waited for before a tile's
-// interactions).
-// Interactions use the hardware v_rsq_f32 (float32); per-tile partial sums are
-// folded into the running total with Kahan compensation when requested; the
-// partitions are reduced through LDS in fixed order (deterministic).
+// Mapping: one workgroup per work item (a target leaf, or a range of its source
+// slots).  Thread t owns one target of the leaf and one source partition.  The
+// leaf's source slots (self leaf first, then the near leaves, each leaf_size
+// slots wide) stream through LDS in tiles; inside a tile partition q takes slots
+// q, q + NPART, ... so the lanes of a partition read one broadcast address per
+// interaction and the tail tile stays balanced.  The next tile's sources are
+// fetched into registers while the current one is consumed, with the near-list
+// entries loaded one tile further ahead than the positions they address (no load
+// is waited for before a tile's interactions).  Per-tile partial sums are folded
+// into the running total with Kahan compensation when requested; the partitions
+// are reduced through LDS in fixed order (deterministic).
+//
+// p2p_kernel takes leaves of 8, 16, 32 and 64 (softened, compensated) with the
+// leaf width known at compile time; p2p_any_kernel everything else.
 
 #include <hip/hip_runtime.h>
 
@@ -40,14 +41,6 @@ static_assert(kP2PLdsBytes * (kP2PBlocksPerCu + 1) > kLdsPerCu && kP2PLdsBytes *
 
 
 template <typename T>
-__device__ __forceinline__ T fast_rsqrt(T x) {
-  if constexpr (sizeof(T) == 4)
-    return __builtin_amdgcn_rsqf(x);
-  else
-    return 1.0 / sqrt(x);
-}
-
-template <typename T>
 __device__ __forceinline__ void kahan_add(T& s, T& c, T v) {
   const T y = v - c;
   const T t = s + y;
@@ -55,61 +48,12 @@ __device__ __forceinline__ void kahan_add(T& s, T& c, T v) {
   s = t;
 }
 
-// Source fetch in two stages.  A target leaf's slot sequence is its own
-// leaf, then its nnear near leaves, leaf_size slots each; thread t owns slots
-// first + l * STRIDE (l < LOADS).  fetch_list loads the raw near-list entries
-// of those slots (indices clamped into range; an empty list reads
-// `fallback`, a valid int32 location, and the value is discarded; no
-// arithmetic on the loaded values, so nothing waits for them here);
-// fetch_positions decodes the same slots with those entries one tile later
-// and loads the positions (slots past `total` or past the last particle are
-// marked invalid and become zero-mass sources).  The P2P loop keeps list
-// loads one tile ahead of position loads, so neither is waited for before the
-// interactions of the current tile.  For leaf_size == WT (power-of-two
-// leaves) the slot decode is a shift and a mask.
-// FIXED: leaf_size == WT, known at compile time (shift and mask, no branch).
-template <int WT, bool FIXED>
-__device__ __forceinline__ void slot_decode(int leaf_size, int slot, int& qi, int& o) {
-  if constexpr (FIXED) {
-    qi = static_cast<int>(static_cast<unsigned>(slot) / WT);
-    o = static_cast<int>(static_cast<unsigned>(slot) % WT);
-  } else {
-    qi = slot / leaf_size;
-    o = slot - qi * leaf_size;
-  }
-}
-
-template <int WT, bool FIXED, int LOADS, int STRIDE>
-__device__ __forceinline__ void fetch_list(int leaf_size, const int32_t* __restrict__ near_list, int nnear,
-                                           const int32_t* __restrict__ fallback, int first, int (&v)[LOADS]) {
-  const int32_t* list = nnear > 0 ? near_list : fallback;
-  const int hi = max(nnear - 1, 0);
-#pragma unroll
-  for (int l = 0; l < LOADS; ++l) {
-    int qi, o;
-    slot_decode<WT, FIXED>(leaf_size, first + l * STRIDE, qi, o);
-    v[l] = list[min(max(qi - 1, 0), hi)];
-  }
-}
-
-template <typename T, int WT, bool FIXED, int LOADS, int STRIDE>
-__device__ __forceinline__ void fetch_positions(const T* __restrict__ pos4, int n, int leaf_size, int leaf, int total,
-                                                int first, const int (&v)[LOADS], V4<T> (&out)[LOADS],
-                                                bool (&valid)[LOADS]) {
-#pragma unroll
-  for (int l = 0; l < LOADS; ++l) {
-    int qi, o;
-    slot_decode<WT, FIXED>(leaf_size, first + l * STRIDE, qi, o);
-    const int sl = qi > 0 ? v[l] : leaf;
-    const int g = first + l * STRIDE < total ? sl * leaf_size + o : n;
-    valid[l] = g < n;
-    out[l] = load4(pos4, min(g, n - 1));
-  }
-}
-
-// Leaf-granular fetch (power-of-two leaves, leaf_size == WT): thread t takes
-// the LOADS consecutive slots first .. first + LOADS - 1, which lie in one
-// source leaf, so one near-list entry and one slot decode serve them all.
+// Leaf-granular fetch (leaf_size == WT, a power of two): thread t takes the LOADS
+// consecutive slots first .. first + LOADS - 1, which lie in one source leaf, so
+// one near-list entry and one slot decode serve them all.  fetch_list_leaf loads
+// the entry (index clamped into range; an empty list reads `fallback`, a valid
+// int32 location, and the value is discarded); the positions are loaded one tile
+// later (slots past `total` or past the last particle become zero-mass sources).
 template <int WT>
 __device__ __forceinline__ int fetch_list_leaf(const int32_t* __restrict__ near_list, int nnear,
                                                const int32_t* __restrict__ fallback, int first) {
@@ -175,6 +119,37 @@ struct P2PItems {
   int32_t num_part;  // rows of partials (items with part >= num_part write nothing)
 };
 
+// Writes one target's sums: partial row of a split leaf, or output row (self
+// potential removed, scaled by G).
+template <typename T, bool POT>
+__device__ __forceinline__ void put_sums(V4<T> r, T mass, int first, int i, int leaf_size, int part_out, T eps2, T G,
+                                         const int32_t* __restrict__ out_index, T* __restrict__ acc,
+                                         T* __restrict__ pot, int32_t accumulate, const P2PItems<T>& items) {
+  if (part_out >= 0) {
+    if (part_out >= items.num_part) return;
+    T* dst = items.partials + (static_cast<int64_t>(part_out) * leaf_size + i) * 4;
+    dst[0] = r.x;
+    dst[1] = r.y;
+    dst[2] = r.z;
+    dst[3] = r.w;
+    return;
+  }
+  T ap = r.w;
+  if (POT && eps2 > T(0)) ap -= mass * fast_rsqrt(eps2);  // remove the softened self term
+  const int64_t row = out_index ? out_index[first + i] : first + i;
+  if (accumulate) {
+    acc[3 * row + 0] += G * r.x;
+    acc[3 * row + 1] += G * r.y;
+    acc[3 * row + 2] += G * r.z;
+    if (POT) pot[row] += -G * ap;
+  } else {
+    acc[3 * row + 0] = G * r.x;
+    acc[3 * row + 1] = G * r.y;
+    acc[3 * row + 2] = G * r.z;
+    if (POT) pot[row] = -G * ap;
+  }
+}
+
 // Workgroup size of the float32 leaf-granular path for leaves of 8: 128
 // threads (16 source partitions), so each thread runs 64 interactions per
 // 1024-source tile and the per-item set-up and partition reduction are shared
@@ -189,28 +164,29 @@ constexpr int kNarrowThreads = JFM_P2P_NARROW_THREADS;
 #define JFM_P2P_NARROW_BLOCKS_PER_CU 8
 #endif
 
-// SAFE: guard r^2 == 0 (unsoftened self term / coincident points).
-// THREADS: workgroup size (kThreads, or kNarrowThreads for narrow leaves).
-template <typename T, int WT, bool POT, bool COMP, bool SAFE, bool FIXED, int THREADS>
-__global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4, int32_t n, int32_t leaf_size,
+// Softened, compensated, leaf_size == WT (the compile-time slot decode and the
+// leaf-granular fetch).  THREADS: workgroup size (kThreads, or kNarrowThreads for
+// narrow leaves).
+template <typename T, int WT, bool POT, int THREADS>
+__global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4, int32_t n,
                                                       const int32_t* __restrict__ near_off,
                                                       const int32_t* __restrict__ near_src, T eps2, T G,
                                                       const int32_t* __restrict__ out_index, T* __restrict__ acc,
                                                       T* __restrict__ pot, int32_t accumulate, P2PItems<T> items) {
+  constexpr int leaf_size = WT;
   constexpr int NPART = THREADS / WT;
   constexpr int TILE = sizeof(T) == 4 ? 1024 : 512;
   constexpr int LOADS = TILE / THREADS;
   static_assert(2 * THREADS <= TILE, "reduction buffer must fit in the tile");
-  // REMAP: leaf-granular fetch; slot s of a tile is stored at
-  // (s % LOADS) * ROW + s / LOADS, so the fetching thread writes its LOADS
+  // Slot s of a tile is stored at (s % LOADS) * ROW + s / LOADS, so the fetching thread writes its LOADS
   // slots to LOADS conflict-free rows and partition p still reads one address
   // per interaction, (p % LOADS) * ROW + p / LOADS + k * NPART / LOADS.  Rows
   // are padded so that the eight partitions a wave reads fall in distinct
   // 4-bank groups: with LOADS = 4 they sit in rows p % 4 at columns p / 4
   // (ROW = THREADS + 2), with LOADS = 8 in rows p at column 0 (ROW = THREADS + 1).
-  constexpr bool REMAP = FIXED && (NPART % LOADS == 0);
-  constexpr bool BUF = REMAP && sizeof(T) == 4;  // float32: buffer-resource fetch
-  constexpr int ROW = REMAP ? THREADS + (LOADS == 8 ? 1 : 2) : THREADS;
+  static_assert(NPART % LOADS == 0, "partitions must cover the tile's rows evenly");
+  constexpr bool BUF = sizeof(T) == 4;  // float32: buffer-resource fetch
+  constexpr int ROW = THREADS + (LOADS == 8 ? 1 : 2);
   // The tile array is padded so that at most kBlocksPerCu workgroups share a
   // CU: the rest of its registers and LDS stay free for the tree-pass kernels
   // that run beside P2P in an overlapped step (at full occupancy their small
@@ -244,24 +220,18 @@ __global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4
   // interaction loop.
   V4<T> next[LOADS];
   bool ok[LOADS];
-  int lst[LOADS];  // near-list entries of the tile after `next`
+  int lst;  // near-list entry of the tile after `next`
   const int tid = threadIdx.x;
   const __amdgpu_buffer_rsrc_t rsrc = pos4_rsrc(pos4, BUF ? n : 0);  // used by the float32 fetch only
-  if constexpr (REMAP) {
-    lst[0] = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, start + LOADS * tid);
-    if constexpr (BUF)
-      fetch_positions_buf<WT, LOADS>(rsrc, n, leaf, total, start + LOADS * tid, lst[0],
-                                     reinterpret_cast<V4<float>(&)[LOADS]>(next));
-    else
-      fetch_positions_leaf<T, WT, LOADS>(pos4, n, leaf, total, start + LOADS * tid, lst[0], next, ok);
-    lst[0] = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, start + TILE + LOADS * tid);
-  } else {
-    fetch_list<WT, FIXED, LOADS, THREADS>(leaf_size, near_src + nb, nsl - 1, near_off, start + tid, lst);
-    fetch_positions<T, WT, FIXED, LOADS, THREADS>(pos4, n, leaf_size, leaf, total, start + tid, lst, next, ok);
-    fetch_list<WT, FIXED, LOADS, THREADS>(leaf_size, near_src + nb, nsl - 1, near_off, start + TILE + tid, lst);
-  }
-  const int rbase = REMAP ? (part % LOADS) * ROW + part / LOADS : part;
-  constexpr int RSTEP = REMAP ? NPART / LOADS : NPART;
+  lst = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, start + LOADS * tid);
+  if constexpr (BUF)
+    fetch_positions_buf<WT, LOADS>(rsrc, n, leaf, total, start + LOADS * tid, lst,
+                                   reinterpret_cast<V4<float>(&)[LOADS]>(next));
+  else
+    fetch_positions_leaf<T, WT, LOADS>(pos4, n, leaf, total, start + LOADS * tid, lst, next, ok);
+  lst = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, start + TILE + LOADS * tid);
+  const int rbase = (part % LOADS) * ROW + part / LOADS;
+  constexpr int RSTEP = NPART / LOADS;
 
   T sx = 0, sy = 0, sz = 0, sp = 0;
   T kx = 0, ky = 0, kz = 0, kp = 0;
@@ -276,19 +246,12 @@ __global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4
     __syncthreads();
     // unconditional (past the end they yield invalid slots): a branch here
     // would make the compiler wait for the loads at its join
-    if constexpr (BUF) {
-      fetch_positions_buf<WT, LOADS>(rsrc, n, leaf, total, base + TILE + LOADS * tid, lst[0],
+    if constexpr (BUF)
+      fetch_positions_buf<WT, LOADS>(rsrc, n, leaf, total, base + TILE + LOADS * tid, lst,
                                      reinterpret_cast<V4<float>(&)[LOADS]>(next));
-      lst[0] = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, base + 2 * TILE + LOADS * tid);
-    } else if constexpr (REMAP) {
-      fetch_positions_leaf<T, WT, LOADS>(pos4, n, leaf, total, base + TILE + LOADS * tid, lst[0], next, ok);
-      lst[0] = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, base + 2 * TILE + LOADS * tid);
-    } else {
-      fetch_positions<T, WT, FIXED, LOADS, THREADS>(pos4, n, leaf_size, leaf, total, base + TILE + tid, lst, next,
-                                                    ok);
-      fetch_list<WT, FIXED, LOADS, THREADS>(leaf_size, near_src + nb, nsl - 1, near_off, base + 2 * TILE + tid,
-                                            lst);
-    }
+    else
+      fetch_positions_leaf<T, WT, LOADS>(pos4, n, leaf, total, base + TILE + LOADS * tid, lst, next, ok);
+    lst = fetch_list_leaf<WT>(near_src + nb, nsl - 1, near_off, base + 2 * TILE + LOADS * tid);
     // Slots past `total` hold zero-mass sources, so every partition runs the
     // same (wave-uniform, scalar-controlled) trip count.
     const int trips = (min(TILE, total - base) + NPART - 1) / NPART;
@@ -300,8 +263,135 @@ __global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4
       const T dy = s.y - xi.y;
       const T dz = s.z - xi.z;
       const T r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
+      const T rinv = fast_rsqrt(r2);
+      const T mr = s.w * rinv;
+      const T mr3 = mr * (rinv * rinv);
+      tx = fma(mr3, dx, tx);
+      ty = fma(mr3, dy, ty);
+      tz = fma(mr3, dz, tz);
+      if (POT) tp += mr;
+    }
+    kahan_add(sx, kx, tx);
+    kahan_add(sy, ky, ty);
+    kahan_add(sz, kz, tz);
+    if (POT) kahan_add(sp, kp, tp);
+  }
+  // partitions reduced pairwise in LDS (fixed tree order, every thread takes part)
+  __syncthreads();
+  tile[threadIdx.x] = V4<T>{sx - kx, sy - ky, sz - kz, sp - kp};
+  __syncthreads();
+#pragma unroll
+  for (int w = NPART / 2; w >= 1; w >>= 1) {
+    if (part < w) {
+      const V4<T> a = tile[threadIdx.x];
+      const V4<T> b = tile[threadIdx.x + w * WT];
+      tile[threadIdx.x] = V4<T>{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
+    }
+    __syncthreads();
+  }
+  if (part == 0 && i < cnt)
+    put_sums<T, POT>(tile[i], xi.w, first, i, leaf_size, part_out, eps2, G, out_index, acc, pot, accumulate, items);
+}
+
+// Any leaf width (1..256), softening and summation.  Thread t owns target
+// t % leaf_size and partition t / leaf_size of floor(256 / leaf_size): with the
+// width rounded up to a power of two instead, leaves of 24 left a quarter of the
+// lanes idle.  A tile's first slot is divided by the width once (the same for the
+// workgroup) and the threads' slots by a multiplication with its reciprocal, exact
+// for the at most kThreads + TILE slots of a tile (magic = ceil(2^32 / leaf_size)).
+// Tiles hold tile_slots <= TILE slots, a multiple of 8 rounds of the partitions
+// where they are few, so that full tiles have no remainder of the unrolled loop.
+// 100k bodies, leaf 24, with potentials: 416 -> 318 us.
+template <typename T, bool POT, bool COMP, bool SAFE>
+__global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__ pos4, int32_t n, int32_t leaf_size,
+                                                           uint32_t magic, int32_t tile_slots,
+                                                           const int32_t* __restrict__ near_off,
+                                                           const int32_t* __restrict__ near_src, T eps2, T G,
+                                                           const int32_t* __restrict__ out_index,
+                                                           T* __restrict__ acc, T* __restrict__ pot,
+                                                           int32_t accumulate, P2PItems<T> items) {
+  constexpr int TILE = sizeof(T) == 4 ? 1024 : 512;
+  constexpr int LOADS = TILE / kThreads;
+  // past the tile's slots: massless rows for the last round of every partition
+  constexpr int kElems = TILE + kThreads;
+  constexpr int kPadElems = static_cast<int>(kP2PLdsBytes / sizeof(V4<T>));
+  __shared__ V4<T> tile[kElems > kPadElems ? kElems : kPadElems];
+  const int tid = threadIdx.x;
+  const int item = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int leaf = items.leaf ? items.leaf[item] : item;
+  auto quotient = [&](uint32_t v) { return leaf_size == 1 ? v : __umulhi(v, magic); };
+  const int npart = kThreads / leaf_size;
+  int part = static_cast<int>(quotient(tid));
+  const int i = tid - part * leaf_size;
+  const bool idle = part >= npart;
+  if (idle) part = 0;  // stays in step with the others, its sums are dropped
+  const int first = leaf * leaf_size;
+  const int cnt = min(leaf_size, n - first);
+  const V4<T> xi = load4(pos4, first + (i < cnt ? i : 0));
+  const int nb = near_off[leaf];
+  const int nsl = 1 + (near_off[leaf + 1] - nb);
+  const int start = items.leaf ? items.s0[item] : 0;
+  const int total = items.leaf ? items.s1[item] : nsl * leaf_size;
+  const int part_out = items.leaf ? items.part[item] : -1;
+  const int32_t* list = nsl > 1 ? near_src + nb : near_off;  // an empty list reads a valid location, unused
+  const int hi = max(nsl - 2, 0);
+
+  V4<T> next[LOADS];
+  bool ok[LOADS];
+  // of the tile after `next`: near-list entries, slots within the source leaf
+  // (complemented for the self leaf)
+  int lst[LOADS], off[LOADS];
+  auto fetch_list = [&](int base) {
+    const int qb = base / leaf_size, ob = base - qb * leaf_size;
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      const uint32_t v = ob + tid + l * kThreads;
+      const int dq = static_cast<int>(quotient(v));
+      const int q = qb + dq, o = static_cast<int>(v) - dq * leaf_size;
+      off[l] = q == 0 ? ~o : o;
+      lst[l] = list[min(max(q - 1, 0), hi)];
+    }
+  };
+  auto fetch_positions = [&](int base) {
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      const bool self = off[l] < 0;
+      const int g = (self ? leaf : lst[l]) * leaf_size + (self ? ~off[l] : off[l]);
+      ok[l] = tid + l * kThreads < min(tile_slots, total - base) && g < n;
+      next[l] = load4(pos4, ok[l] ? g : 0);
+    }
+  };
+  fetch_list(start);
+  fetch_positions(start);
+  fetch_list(start + tile_slots);
+  tile[TILE + tid] = V4<T>{T(0), T(0), T(0), T(0)};
+
+  T sx = 0, sy = 0, sz = 0, sp = 0;
+  T kx = 0, ky = 0, kz = 0, kp = 0;
+  for (int base = start; base < total; base += tile_slots) {
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      V4<T> q = next[l];
+      if (!ok[l]) q.w = T(0);
+      tile[l * kThreads + tid] = q;
+    }
+    __syncthreads();
+    // unconditional, as in p2p_kernel: past the end they yield massless slots
+    fetch_positions(base + tile_slots);
+    fetch_list(base + 2 * tile_slots);
+    const int trips = (min(tile_slots, total - base) + npart - 1) / npart;
+    T tx = 0, ty = 0, tz = 0, tp = 0;
+    const V4<T>* src = tile + part;
+#pragma unroll 8
+    for (int k = 0; k < trips; ++k, src += npart) {
+      const V4<T> s = *src;
+      const T dx = s.x - xi.x;
+      const T dy = s.y - xi.y;
+      const T dz = s.z - xi.z;
+      const T r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
       T rinv = fast_rsqrt(r2);
-      if (SAFE) rinv = r2 > T(0) ? rinv : T(0);
+      if (SAFE) rinv = r2 > T(0) ? rinv : T(0);  // the self pair, coincident points
       const T mr = s.w * rinv;
       const T mr3 = mr * (rinv * rinv);
       tx = fma(mr3, dx, tx);
@@ -321,45 +411,21 @@ __global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4
       if (POT) sp += tp;
     }
   }
-  // partitions reduced pairwise in LDS (fixed tree order, every thread takes part)
   __syncthreads();
-  tile[threadIdx.x] = V4<T>{sx - kx, sy - ky, sz - kz, sp - kp};
+  tile[tid] = V4<T>{sx - kx, sy - ky, sz - kz, sp - kp};
   __syncthreads();
-#pragma unroll
-  for (int w = NPART / 2; w >= 1; w >>= 1) {
-    if (part < w) {
-      const V4<T> a = tile[threadIdx.x];
-      const V4<T> b = tile[threadIdx.x + w * WT];
-      tile[threadIdx.x] = V4<T>{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
+  int w = 1;
+  while (2 * w < npart) w *= 2;  // pairwise over the partitions, fixed order
+  for (; w >= 1; w >>= 1) {
+    if (!idle && part < w && part + w < npart) {
+      const V4<T> a = tile[tid];
+      const V4<T> b = tile[tid + w * leaf_size];
+      tile[tid] = V4<T>{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
     }
     __syncthreads();
   }
-  if (part == 0 && i < cnt) {
-    const V4<T> r = tile[i];
-    T ax = r.x, ay = r.y, az = r.z, ap = r.w;
-    if (part_out >= 0) {
-      if (part_out >= items.num_part) return;
-      T* dst = items.partials + (static_cast<int64_t>(part_out) * leaf_size + i) * 4;
-      dst[0] = ax;
-      dst[1] = ay;
-      dst[2] = az;
-      dst[3] = ap;
-      return;
-    }
-    if (POT && eps2 > T(0)) ap -= xi.w * fast_rsqrt(eps2);  // remove the softened self term
-    const int64_t row = out_index ? out_index[first + i] : first + i;
-    if (accumulate) {
-      acc[3 * row + 0] += G * ax;
-      acc[3 * row + 1] += G * ay;
-      acc[3 * row + 2] += G * az;
-      if (POT) pot[row] += -G * ap;
-    } else {
-      acc[3 * row + 0] = G * ax;
-      acc[3 * row + 1] = G * ay;
-      acc[3 * row + 2] = G * az;
-      if (POT) pot[row] = -G * ap;
-    }
-  }
+  if (!idle && part == 0 && i < cnt)
+    put_sums<T, POT>(tile[i], xi.w, first, i, leaf_size, part_out, eps2, G, out_index, acc, pot, accumulate, items);
 }
 
 // Leaves split over several items: one workgroup per split leaf.  Target i
@@ -412,61 +478,72 @@ __global__ __launch_bounds__(kThreads) void p2p_reduce_kernel(const T* __restric
   }
 }
 
+// Leaves of 8 to 64, softened and compensated, run on the kernel
+// with the width compiled in: at 1M bodies and leaf 16 its fetch takes 35
+// instructions a tile against about 110.  float32 leaves of 8 run in narrow
+// workgroups.  Row offsets of its float32 fetch bound n.
 template <typename T, int WT>
-int32_t launch_p2p_wt(hipStream_t s, const T* pos4, int32_t n, int32_t leaf_size, int32_t num_blocks,
-                      const int32_t* near_off, const int32_t* near_src, T eps2, T G, const int32_t* out_index,
-                      T* acc, T* pot, bool comp, bool accumulate, P2PItems<T> items) {
-  const bool want_pot = pot != nullptr;
-  const bool safe = !(eps2 > T(0));
-  // the common cases (softened, compensated, leaf_size == WT) get the compile-time
-  // slot decode and leaf-granular fetch; every other combination the general one
-  // float32 leaves of 8 on the fast path run in narrow workgroups
+void launch_p2p_wt(hipStream_t s, const T* pos4, int32_t n, int32_t num_blocks, const int32_t* near_off,
+                   const int32_t* near_src, T eps2, T G, const int32_t* out_index, T* acc, T* pot, bool accumulate,
+                   P2PItems<T> items) {
   constexpr int kFastThreads = (sizeof(T) == 4 && WT == 8) ? kNarrowThreads : kThreads;
-#define JFM_P2P_LAUNCH(POT, COMP, SAFE)                                                                      \
-  if (COMP && !SAFE && leaf_size == WT && (sizeof(T) == 8 || n <= kBufMaxRows))                              \
-    p2p_kernel<T, WT, POT, COMP, SAFE, true, kFastThreads><<<num_blocks, kFastThreads, 0, s>>>(              \
-        pos4, n, leaf_size, near_off, near_src, eps2, G, out_index, acc, pot, accumulate ? 1 : 0, items);    \
-  else                                                                                                       \
-    p2p_kernel<T, WT, POT, COMP, SAFE, false, kThreads><<<num_blocks, kThreads, 0, s>>>(                      \
-        pos4, n, leaf_size, near_off, near_src, eps2, G, out_index, acc, pot, accumulate ? 1 : 0, items)
-  if (want_pot) {
-    if (comp) {
-      if (safe) JFM_P2P_LAUNCH(true, true, true); else JFM_P2P_LAUNCH(true, true, false);
-    } else {
-      if (safe) JFM_P2P_LAUNCH(true, false, true); else JFM_P2P_LAUNCH(true, false, false);
-    }
-  } else {
-    if (comp) {
-      if (safe) JFM_P2P_LAUNCH(false, true, true); else JFM_P2P_LAUNCH(false, true, false);
-    } else {
-      if (safe) JFM_P2P_LAUNCH(false, false, true); else JFM_P2P_LAUNCH(false, false, false);
-    }
-  }
-#undef JFM_P2P_LAUNCH
-  return check_launch("jfm_p2p");
+  if (pot)
+    p2p_kernel<T, WT, true, kFastThreads><<<num_blocks, kFastThreads, 0, s>>>(
+        pos4, n, near_off, near_src, eps2, G, out_index, acc, pot, accumulate ? 1 : 0, items);
+  else
+    p2p_kernel<T, WT, false, kFastThreads><<<num_blocks, kFastThreads, 0, s>>>(
+        pos4, n, near_off, near_src, eps2, G, out_index, acc, pot, accumulate ? 1 : 0, items);
+}
+
+template <typename T, bool POT>
+void launch_p2p_any(hipStream_t s, const T* pos4, int32_t n, int32_t leaf_size, int32_t num_blocks,
+                    const int32_t* near_off, const int32_t* near_src, T eps2, T G, const int32_t* out_index, T* acc,
+                    T* pot, bool comp, bool accumulate, P2PItems<T> items) {
+  const bool safe = !(eps2 > T(0));
+  const uint32_t magic = static_cast<uint32_t>(((uint64_t(1) << 32) + leaf_size - 1) / leaf_size);
+  constexpr int kTile = sizeof(T) == 4 ? 1024 : 512;
+  const int npart = kThreads / leaf_size;
+  const int round = npart <= 32 ? 8 * npart : 4 * npart <= kTile ? 4 * npart : npart;
+  const int tile_slots = kTile - kTile % round;
+#define JFM_P2P_ANY(COMP, SAFE)                                                                              \
+  p2p_any_kernel<T, POT, COMP, SAFE><<<num_blocks, kThreads, 0, s>>>(pos4, n, leaf_size, magic, tile_slots, \
+                                                                     near_off, near_src, eps2, G,          \
+                                                                     out_index, acc, pot,                  \
+                                                                     accumulate ? 1 : 0, items)
+  if (comp && safe)
+    JFM_P2P_ANY(true, true);
+  else if (comp)
+    JFM_P2P_ANY(true, false);
+  else if (safe)
+    JFM_P2P_ANY(false, true);
+  else
+    JFM_P2P_ANY(false, false);
+#undef JFM_P2P_ANY
 }
 
 template <typename T>
 int32_t launch_p2p(hipStream_t s, const T* pos4, int32_t n, int32_t leaf_size, int32_t num_leaves,
                    const int32_t* near_off, const int32_t* near_src, T eps2, T G, const int32_t* out_index, T* acc,
                    T* pot, bool comp, bool accumulate, P2PItems<T> items = P2PItems<T>{}) {
-  if (leaf_size <= 8)
-    return launch_p2p_wt<T, 8>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                               pot, comp, accumulate, items);
-  if (leaf_size <= 16)
-    return launch_p2p_wt<T, 16>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                                pot, comp, accumulate, items);
-  if (leaf_size <= 32)
-    return launch_p2p_wt<T, 32>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                                pot, comp, accumulate, items);
-  if (leaf_size <= 64)
-    return launch_p2p_wt<T, 64>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                                pot, comp, accumulate, items);
-  if (leaf_size <= 128)
-    return launch_p2p_wt<T, 128>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                                 pot, comp, accumulate, items);
-  return launch_p2p_wt<T, 256>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc,
-                               pot, comp, accumulate, items);
+  const bool fast = comp && eps2 > T(0) && (sizeof(T) == 8 || n <= kBufMaxRows);
+#define JFM_P2P_WT(WT)                                                                                             \
+  launch_p2p_wt<T, WT>(s, pos4, n, num_leaves, near_off, near_src, eps2, G, out_index, acc, pot, accumulate, items)
+  if (fast && leaf_size == 8)
+    JFM_P2P_WT(8);
+  else if (fast && leaf_size == 16)
+    JFM_P2P_WT(16);
+  else if (fast && leaf_size == 32)
+    JFM_P2P_WT(32);
+  else if (fast && leaf_size == 64)
+    JFM_P2P_WT(64);
+  else if (pot)
+    launch_p2p_any<T, true>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc, pot, comp,
+                            accumulate, items);
+  else
+    launch_p2p_any<T, false>(s, pos4, n, leaf_size, num_leaves, near_off, near_src, eps2, G, out_index, acc, pot,
+                             comp, accumulate, items);
+#undef JFM_P2P_WT
+  return check_launch("jfm_p2p");
 }
 
 }  // namespace
