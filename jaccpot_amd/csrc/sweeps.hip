@@ -206,18 +206,18 @@ __global__ __launch_bounds__(kWave) void p2m_group_kernel(const T* __restrict__ 
 
 // L2L into one node: L += l2l(L_parent, c_parent - c).
 template <typename T, int P>
-__device__ __forceinline__ void l2l_node(int node, const int32_t* __restrict__ parent,
-                                         const T* __restrict__ centers4, T* __restrict__ locals, int32_t cs) {
+__device__ __forceinline__ void l2l_node(int node, int par, const T* __restrict__ centers4,
+                                         T* __restrict__ locals, int32_t cs) {
   constexpr int C = ncoef(P);
-  const int par = parent[node];
   const V4<T> cp = load4(centers4, par);
   const V4<T> cc = load4(centers4, node);
   T v[C];
   load_row<T, C>(locals + static_cast<int64_t>(par) * cs, v);
+  T w[C];
+  if constexpr (P <= kDirectShift) load_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);  // with the parent's
   T u[C];
   l2l<T, P>(v, u, cp.x - cc.x, cp.y - cc.y, cp.z - cc.z);  // source(parent) - destination(child)
-  T w[C];
-  load_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
+  if constexpr (P > kDirectShift) load_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
 #pragma unroll
   for (int j = 0; j < C; ++j) w[j] += u[j];
   store_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
@@ -229,11 +229,10 @@ __device__ __forceinline__ void l2l_node(int node, const int32_t* __restrict__ p
 // left + right and side 0 writes the node.  Halves the dependent instruction
 // chain of a level, which is what a level of the upward pass waits for.
 template <typename T, int P>
-__device__ __forceinline__ void m2m_node(int node, int side, bool live, const int32_t* __restrict__ left,
-                                         const int32_t* __restrict__ right, const int32_t* __restrict__ node_range,
-                                         T* __restrict__ mult, int32_t cs, T* __restrict__ centers4) {
+__device__ __forceinline__ void m2m_node(int node, int lc, int rc, int side, bool live,
+                                         const int32_t* __restrict__ node_range, T* __restrict__ mult, int32_t cs,
+                                         T* __restrict__ centers4) {
   constexpr int C = ncoef(P);
-  const int lc = left[node], rc = right[node];
   const V4<T> cl = load4(centers4, lc);
   const V4<T> cr = load4(centers4, rc);
   const T tot = cl.w + cr.w;
@@ -273,16 +272,24 @@ __global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ 
   // lanes past the level repeat its last node (results dropped) so that both
   // lanes of every pair reach the exchange
   const bool live = (t >> 1) < count;
-  m2m_node<T, P>(nodes[live ? (t >> 1) : count - 1], t & 1, live, left, right, node_range, mult, cs, centers4);
+  const int node = nodes[live ? (t >> 1) : count - 1];
+  m2m_node<T, P>(node, left[node], right[node], t & 1, live, node_range, mult, cs, centers4);
 }
 
 // A run of levels with few nodes each in one workgroup, a barrier between the
 // levels: such a level is one node's dependent chain (loads, about 300 VALU
 // instructions at order 4) on a nearly empty GPU, and as a launch of its own it
-// also pays the start and drain of a kernel and the host's call.  256 threads,
-// one wave per SIMD, so that the workgroup finds room on a CU beside the P2P's
-// workgroups (wider ones wait for several of those to end).
+// also pays the start and drain of a kernel and the host's call.  What does not
+// depend on the level before is loaded ahead: the node numbers two levels early,
+// their relatives one level early, so a level waits for one round of loads.  256
+// threads, one wave per SIMD, so that the workgroup finds room on a CU beside the
+// P2P's workgroups (wider ones wait for several of those to end).
 constexpr int kSpanThreads = 256;
+
+// First entry of a thread in level `lev` of a span (-1: none).
+__device__ __forceinline__ int span_first(const LevelSpan& span, int lev, int k) {
+  return lev < span.n && span.off[lev] + k < span.off[lev + 1] ? span.off[lev] + k : -1;
+}
 
 template <typename T, int P>
 __global__ __launch_bounds__(kSpanThreads) void m2m_span_kernel(const int32_t* __restrict__ nodes, LevelSpan span,
@@ -291,10 +298,24 @@ __global__ __launch_bounds__(kSpanThreads) void m2m_span_kernel(const int32_t* _
                                                                 const int32_t* __restrict__ node_range,
                                                                 T* __restrict__ mult, int32_t cs,
                                                                 T* __restrict__ centers4) {
+  const int slot = threadIdx.x >> 1;  // both lanes of a pair stay together
+  const int k0 = span_first(span, 0, slot), k1 = span_first(span, 1, slot);
+  int node = nodes[max(k0, span.off[0])], next = nodes[max(k1, span.off[0])];
+  int lc = left[node], rc = right[node];
   for (int lev = 0; lev < span.n; ++lev) {
-    const int b = span.off[lev], e = span.off[lev + 1];
-    for (int k = b + (threadIdx.x >> 1); k < e; k += kSpanThreads / 2)  // both lanes of a pair stay together
-      m2m_node<T, P>(nodes[k], threadIdx.x & 1, true, left, right, node_range, mult, cs, centers4);
+    const int next2 = nodes[max(span_first(span, lev + 2, slot), span.off[0])];
+    const int lc1 = left[next], rc1 = right[next];
+    int k = span_first(span, lev, slot);
+    if (k >= 0) {
+      m2m_node<T, P>(node, lc, rc, threadIdx.x & 1, true, node_range, mult, cs, centers4);
+      for (k += kSpanThreads / 2; k < span.off[lev + 1]; k += kSpanThreads / 2)
+        m2m_node<T, P>(nodes[k], left[nodes[k]], right[nodes[k]], threadIdx.x & 1, true, node_range, mult, cs,
+                       centers4);
+    }
+    node = next;
+    next = next2;
+    lc = lc1;
+    rc = rc1;
     __syncthreads();
   }
 }
@@ -305,9 +326,22 @@ __global__ __launch_bounds__(kSpanThreads) void l2l_span_kernel(const int32_t* _
                                                                 const int32_t* __restrict__ parent,
                                                                 const T* __restrict__ centers4,
                                                                 T* __restrict__ locals, int32_t cs) {
+  const int slot = threadIdx.x;
+  const int k0 = span_first(span, 0, slot), k1 = span_first(span, 1, slot);
+  int node = nodes[max(k0, span.off[0])], next = nodes[max(k1, span.off[0])];
+  int par = parent[node];
   for (int lev = 0; lev < span.n; ++lev) {
-    for (int k = span.off[lev] + threadIdx.x; k < span.off[lev + 1]; k += kSpanThreads)
-      l2l_node<T, P>(nodes[k], parent, centers4, locals, cs);
+    const int next2 = nodes[max(span_first(span, lev + 2, slot), span.off[0])];
+    const int par1 = parent[next];
+    int k = span_first(span, lev, slot);
+    if (k >= 0) {
+      l2l_node<T, P>(node, par, centers4, locals, cs);
+      for (k += kSpanThreads; k < span.off[lev + 1]; k += kSpanThreads)
+        l2l_node<T, P>(nodes[k], parent[nodes[k]], centers4, locals, cs);
+    }
+    node = next;
+    next = next2;
+    par = par1;
     __syncthreads();
   }
 }
@@ -324,7 +358,7 @@ __global__ __launch_bounds__(kWave) void l2l_kernel(const int32_t* __restrict__ 
                                                     int32_t cs) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= count) return;
-  l2l_node<T, P>(nodes[t], parent, centers4, locals, cs);
+  l2l_node<T, P>(nodes[t], parent[nodes[t]], centers4, locals, cs);
 }
 
 // One thread per particle: far field from its leaf's local expansion.
