@@ -10,6 +10,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_math.hpp"
 #include "launch.hpp"
 #include "rows.hpp"
@@ -223,6 +225,26 @@ __device__ __forceinline__ void l2l_node(int node, int par, const T* __restrict_
   store_row<T, C>(locals + static_cast<int64_t>(node) * cs, w);
 }
 
+// Centre and mass of the node with children lc, rc.
+template <typename T>
+__device__ __forceinline__ V4<T> join_centers(V4<T> cl, V4<T> cr, int lc, int rc,
+                                              const int32_t* __restrict__ node_range) {
+  V4<T> c;
+  c.w = cl.w + cr.w;
+  if (c.w > T(0)) {
+    c.x = (cl.w * cl.x + cr.w * cr.x) / c.w;
+    c.y = (cl.w * cl.y + cr.w * cr.y) / c.w;
+    c.z = (cl.w * cl.z + cr.w * cr.z) / c.w;
+  } else {  // massless: particle-count-weighted mean of the children's means
+    const T nl = static_cast<T>(node_range[2 * lc + 1] - node_range[2 * lc] + 1);
+    const T nr = static_cast<T>(node_range[2 * rc + 1] - node_range[2 * rc] + 1);
+    c.x = (nl * cl.x + nr * cr.x) / (nl + nr);
+    c.y = (nl * cl.y + nr * cr.y) / (nl + nr);
+    c.z = (nl * cl.z + nr * cr.z) / (nl + nr);
+  }
+  return c;
+}
+
 // Two lanes per internal node of a level (children already done): the lane of
 // side 0 translates the left child's multipole to the node's centre of mass, the
 // lane of side 1 (its neighbour t ^ 1) the right one's; the sum is formed as
@@ -235,30 +257,18 @@ __device__ __forceinline__ void m2m_node(int node, int lc, int rc, int side, boo
   constexpr int C = ncoef(P);
   const V4<T> cl = load4(centers4, lc);
   const V4<T> cr = load4(centers4, rc);
-  const T tot = cl.w + cr.w;
-  T cx, cy, cz;
-  if (tot > T(0)) {
-    cx = (cl.w * cl.x + cr.w * cr.x) / tot;
-    cy = (cl.w * cl.y + cr.w * cr.y) / tot;
-    cz = (cl.w * cl.z + cr.w * cr.z) / tot;
-  } else {  // massless: particle-count-weighted mean of the children's means
-    const T nl = static_cast<T>(node_range[2 * lc + 1] - node_range[2 * lc] + 1);
-    const T nr = static_cast<T>(node_range[2 * rc + 1] - node_range[2 * rc] + 1);
-    cx = (nl * cl.x + nr * cr.x) / (nl + nr);
-    cy = (nl * cl.y + nr * cr.y) / (nl + nr);
-    cz = (nl * cl.z + nr * cr.z) / (nl + nr);
-  }
+  const V4<T> c = join_centers(cl, cr, lc, rc, node_range);
   const int ch = side == 0 ? lc : rc;
   const V4<T> cc = side == 0 ? cl : cr;
   T v[C];
   load_row<T, C>(mult + static_cast<int64_t>(ch) * cs, v);
   T w[C];
-  m2m<T, P>(v, w, cc.x - cx, cc.y - cy, cc.z - cz);  // source - destination
+  m2m<T, P>(v, w, cc.x - c.x, cc.y - c.y, cc.z - c.z);  // source - destination
 #pragma unroll
   for (int j = 0; j < C; ++j) w[j] = w[j] + dpp_get<0xB1>(w[j]);  // left + right on both lanes
   if (side == 0 && live) {
     store_row<T, C>(mult + static_cast<int64_t>(node) * cs, w);
-    store4(centers4, node, V4<T>{cx, cy, cz, tot});
+    store4(centers4, node, c);
   }
 }
 
@@ -284,11 +294,92 @@ __global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ 
 // their relatives one level early, so a level waits for one round of loads.  256
 // threads, one wave per SIMD, so that the workgroup finds room on a CU beside the
 // P2P's workgroups (wider ones wait for several of those to end).
+//
+// From order 6 a level of at most a wave's nodes is cut four ways: each wave
+// computes a quarter of every node's outputs (shift_part) by the direct form, 445
+// instructions instead of 1080.  Such a level takes 1.8 us instead of 3.1 at order
+// 6, 3.0 instead of 5.2 at order 8 (float32, upward, 16 nodes; without arithmetic
+// 0.65).  Below, and for wider levels, the four-byte accesses of the parts cost
+// more than that saves (order 4: 1.3 us either way; 100 nodes at order 6: 7.0
+// against 3.8).
 constexpr int kSpanThreads = 256;
+constexpr int kPartOrder = 6;
 
 // First entry of a thread in level `lev` of a span (-1: none).
 __device__ __forceinline__ int span_first(const LevelSpan& span, int lev, int k) {
   return lev < span.n && span.off[lev] + k < span.off[lev + 1] ? span.off[lev] + k : -1;
+}
+
+// One of the four parts of a node's M2M (lanes as in m2m_node; both lanes of a pair live).
+template <typename T, int P, int PART>
+__device__ __forceinline__ void m2m_node_part(int node, int lc, int rc, int side,
+                                              const int32_t* __restrict__ node_range, T* __restrict__ mult,
+                                              int32_t cs, T* __restrict__ centers4) {
+  constexpr int C = ncoef(P);
+  const V4<T> cl = load4(centers4, lc);
+  const V4<T> cr = load4(centers4, rc);
+  T v[C];
+  load_row<T, C>(mult + static_cast<int64_t>(side == 0 ? lc : rc) * cs, v);
+  const V4<T> c = join_centers(cl, cr, lc, rc, node_range);
+  const V4<T> cc = side == 0 ? cl : cr;
+  T w[C];
+  shift_part_of<T, P, true, PART>(v, w, cc.x - c.x, cc.y - c.y, cc.z - c.z);  // source - destination
+  T* row = mult + static_cast<int64_t>(node) * cs;
+#pragma unroll
+  for (int n = 0; n <= P; ++n)
+#pragma unroll
+    for (int m = -n; m <= n; ++m)
+      if (in_part<PART>(m < 0 ? -m : m)) {
+        const int j = sh_idx(n, m);
+        const T sum = w[j] + dpp_get<0xB1>(w[j]);  // left + right
+        if (side == 0) row[j] = sum;
+      }
+  if (PART == 3 && side == 0) {
+    for (int j = C; j < cs; ++j) row[j] = T(0);
+    store4(centers4, node, c);
+  }
+}
+
+// One of the four parts of a node's L2L.
+template <typename T, int P, int PART>
+__device__ __forceinline__ void l2l_node_part(int node, int par, const T* __restrict__ centers4,
+                                              T* __restrict__ locals, int32_t cs) {
+  constexpr int C = ncoef(P);
+  const V4<T> cp = load4(centers4, par);
+  const V4<T> cc = load4(centers4, node);
+  T v[C];
+  load_row<T, C>(locals + static_cast<int64_t>(par) * cs, v);
+  T* row = locals + static_cast<int64_t>(node) * cs;
+  T u[C], w[C];
+#pragma unroll
+  for (int n = 0; n <= P; ++n)
+#pragma unroll
+    for (int m = -n; m <= n; ++m)
+      if (in_part<PART>(m < 0 ? -m : m)) u[sh_idx(n, m)] = row[sh_idx(n, m)];
+  shift_part_of<T, P, false, PART>(v, w, cp.x - cc.x, cp.y - cc.y, cp.z - cc.z);  // source - destination
+#pragma unroll
+  for (int n = 0; n <= P; ++n)
+#pragma unroll
+    for (int m = -n; m <= n; ++m)
+      if (in_part<PART>(m < 0 ? -m : m)) row[sh_idx(n, m)] = u[sh_idx(n, m)] + w[sh_idx(n, m)];
+}
+
+// f(std::integral_constant<int, part>) for this wave's part (the same for the wave).
+template <typename F>
+__device__ __forceinline__ void for_wave_part(F f) {
+  switch (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) {
+    case 0: f(std::integral_constant<int, 0>()); break;
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    default: f(std::integral_constant<int, 3>());
+  }
+}
+static_assert(kSpanThreads == 4 * kWave, "one wave for each part");
+
+// Whether a level of `count` nodes (`lanes` lanes each) runs in parts.
+template <int P>
+__device__ __forceinline__ bool by_parts(int count, int lanes) {
+  return P >= kPartOrder && count * lanes <= kWave;
 }
 
 template <typename T, int P>
@@ -298,15 +389,24 @@ __global__ __launch_bounds__(kSpanThreads) void m2m_span_kernel(const int32_t* _
                                                                 const int32_t* __restrict__ node_range,
                                                                 T* __restrict__ mult, int32_t cs,
                                                                 T* __restrict__ centers4) {
-  const int slot = threadIdx.x >> 1;  // both lanes of a pair stay together
-  const int k0 = span_first(span, 0, slot), k1 = span_first(span, 1, slot);
-  int node = nodes[max(k0, span.off[0])], next = nodes[max(k1, span.off[0])];
+  // this thread's first entry of a level (both lanes of a pair stay together)
+  auto first = [&](int lev) {
+    const bool parts = lev < span.n && by_parts<P>(span.off[lev + 1] - span.off[lev], 2);
+    return span_first(span, lev, (parts ? threadIdx.x % kWave : threadIdx.x) / 2);
+  };
+  int node = nodes[max(first(0), span.off[0])], next = nodes[max(first(1), span.off[0])];
   int lc = left[node], rc = right[node];
   for (int lev = 0; lev < span.n; ++lev) {
-    const int next2 = nodes[max(span_first(span, lev + 2, slot), span.off[0])];
+    const int next2 = nodes[max(first(lev + 2), span.off[0])];
     const int lc1 = left[next], rc1 = right[next];
-    int k = span_first(span, lev, slot);
-    if (k >= 0) {
+    int k = first(lev);
+    if (by_parts<P>(span.off[lev + 1] - span.off[lev], 2)) {
+      if constexpr (P >= kPartOrder)
+        for_wave_part([&](auto part) {
+          if (k >= 0)
+            m2m_node_part<T, P, decltype(part)::value>(node, lc, rc, threadIdx.x & 1, node_range, mult, cs, centers4);
+        });
+    } else if (k >= 0) {
       m2m_node<T, P>(node, lc, rc, threadIdx.x & 1, true, node_range, mult, cs, centers4);
       for (k += kSpanThreads / 2; k < span.off[lev + 1]; k += kSpanThreads / 2)
         m2m_node<T, P>(nodes[k], left[nodes[k]], right[nodes[k]], threadIdx.x & 1, true, node_range, mult, cs,
@@ -326,15 +426,22 @@ __global__ __launch_bounds__(kSpanThreads) void l2l_span_kernel(const int32_t* _
                                                                 const int32_t* __restrict__ parent,
                                                                 const T* __restrict__ centers4,
                                                                 T* __restrict__ locals, int32_t cs) {
-  const int slot = threadIdx.x;
-  const int k0 = span_first(span, 0, slot), k1 = span_first(span, 1, slot);
-  int node = nodes[max(k0, span.off[0])], next = nodes[max(k1, span.off[0])];
+  auto first = [&](int lev) {
+    const bool parts = lev < span.n && by_parts<P>(span.off[lev + 1] - span.off[lev], 1);
+    return span_first(span, lev, parts ? threadIdx.x % kWave : threadIdx.x);
+  };
+  int node = nodes[max(first(0), span.off[0])], next = nodes[max(first(1), span.off[0])];
   int par = parent[node];
   for (int lev = 0; lev < span.n; ++lev) {
-    const int next2 = nodes[max(span_first(span, lev + 2, slot), span.off[0])];
+    const int next2 = nodes[max(first(lev + 2), span.off[0])];
     const int par1 = parent[next];
-    int k = span_first(span, lev, slot);
-    if (k >= 0) {
+    int k = first(lev);
+    if (by_parts<P>(span.off[lev + 1] - span.off[lev], 1)) {
+      if constexpr (P >= kPartOrder)
+        for_wave_part([&](auto part) {
+          if (k >= 0) l2l_node_part<T, P, decltype(part)::value>(node, par, centers4, locals, cs);
+        });
+    } else if (k >= 0) {
       l2l_node<T, P>(node, par, centers4, locals, cs);
       for (k += kSpanThreads; k < span.off[lev + 1]; k += kSpanThreads)
         l2l_node<T, P>(nodes[k], parent[nodes[k]], centers4, locals, cs);

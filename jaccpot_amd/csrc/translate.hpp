@@ -223,9 +223,19 @@ __host__ __device__ __forceinline__ void m2l(T* v, T* w, T dx, T dy, T dz) {
   }
 }
 
+// A shift's outputs in four parts of nearly equal work, by order |m|: {1, 7}, {2, 6},
+// {3, 5}, {0, 4, 8} (20, 20, 20 and 21 of the 81 outputs at order 8, 12, 12, 12 and
+// 13 of 49 at order 6).
+__host__ __device__ constexpr int shift_part(int m) { return m == 0 || m == 4 || m == 8 ? 3 : (m < 4 ? m : 8 - m) - 1; }
+// Whether part PART (-1: all of them) computes outputs of order m.
+template <int PART>
+__host__ __device__ constexpr bool in_part(int m) {
+  return PART < 0 || shift_part(m) == PART;
+}
+
 // Contributions of degree N of the regular harmonics to w.  UP: M2M (input
-// degree k, output degree N + k); else L2L, its transpose.
-template <typename T, int P, bool UP, int N>
+// degree k, output degree N + k); else L2L, its transpose.  Only outputs of PART.
+template <typename T, int P, bool UP, int N, int PART = -1>
 __host__ __device__ __forceinline__ void shift_degrees(const T* v, T* w, T x, T y, T z, T r2, const T* c1,
                                                        const T* s1, const T* c2, const T* s2) {
   if constexpr (N <= P) {
@@ -233,7 +243,10 @@ __host__ __device__ __forceinline__ void shift_degrees(const T* v, T* w, T x, T 
     regular_degree<T, N>(x, y, z, r2, c1, s1, c2, s2, c, s);
     if constexpr (N == 0) {
 #pragma unroll
-      for (int j = 0; j < ncoef(P); ++j) w[j] = v[j];
+      for (int n = 0; n <= P; ++n)
+#pragma unroll
+        for (int m = -n; m <= n; ++m)
+          if (in_part<PART>(m < 0 ? -m : m)) w[sh_idx(n, m)] = v[sh_idx(n, m)];
     } else {
       // rows: the higher degree n = N + k with order m, columns: degree k with order l
 #pragma unroll
@@ -241,7 +254,7 @@ __host__ __device__ __forceinline__ void shift_degrees(const T* v, T* w, T x, T 
 #pragma unroll
         for (int l = 0; l <= P - N; ++l) {
           const int dm = m >= l ? m - l : l - m;
-          if (dm > N) continue;
+          if (dm > N || !in_part<PART>(UP ? m : l)) continue;
           const bool sum = m + l <= N;
           const T sg = (l & 1) ? T(-1) : T(1);
           const T fl = (m < l && (dm & 1)) ? T(-1) : T(1);
@@ -286,8 +299,15 @@ __host__ __device__ __forceinline__ void shift_degrees(const T* v, T* w, T x, T 
           }
         }
     }
-    shift_degrees<T, P, UP, N + 1>(v, w, x, y, z, r2, c, s, c1, s1);
+    shift_degrees<T, P, UP, N + 1, PART>(v, w, x, y, z, r2, c, s, c1, s1);
   }
+}
+
+// One part of w = m2m(v, d) (UP) or l2l(v, d), direct at every order.
+template <typename T, int P, bool UP, int PART>
+__host__ __device__ __forceinline__ void shift_part_of(const T* v, T* w, T dx, T dy, T dz) {
+  const T zero[1] = {T(0)};
+  shift_degrees<T, P, UP, 0, PART>(v, w, dx, dy, dz, fma(dx, dx, fma(dy, dy, dz * dz)), zero, zero, zero, zero);
 }
 
 // w = m2m(v, d), d = source - destination.  Direct up to order kDirectShift: 258 /
