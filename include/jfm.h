@@ -419,9 +419,14 @@ int32_t jfm_evaluate(void* stream, int32_t dtype, int32_t p, const void* pos4, i
  * pairs; other rows must be zero), L2L levels, jfm_com_chain (chain
  * [L][8]), jfm_leaf_adjoint_b (P2M adjoint + centre-of-mass chain, writes
  * gpos [rows][3], gmass [rows] at out_index). */
+/* flags [L]: 1 where a leaf's records of v4 [N][4] are not all zero.  Taken on
+ * cot4 it is the `active` argument of the adjoint P2P entry points (NULL: every
+ * leaf): pairs of two inactive leaves contribute exact zeros and are skipped. */
+int32_t jfm_leaf_nonzero(void* stream, int32_t dtype, const void* v4, int32_t n, int32_t num_leaves,
+                         int32_t leaf_size, uint8_t* flags);
 int32_t jfm_p2p_adjoint(void* stream, int32_t dtype, const void* pos4, const void* cot4, int32_t n,
                         int32_t num_leaves, int32_t leaf_size, const int32_t* near_off, const int32_t* near_src,
-                        double eps2, double G, void* grad4);
+                        const uint8_t* active, double eps2, double G, void* grad4);
 /* jfm_p2p_adjoint over the work items of jfm_p2p_items (same item arrays):
  * single-item leaves store their grad4 rows, split leaves leave partials that
  * jfm_p2p_adjoint_reduce adds in item order and stores. */
@@ -429,6 +434,7 @@ int32_t jfm_p2p_adjoint_items(void* stream, int32_t dtype, const void* pos4, con
                               int32_t num_leaves, int32_t leaf_size, int32_t num_items, const int32_t* item_leaf,
                               const int32_t* item_s0, const int32_t* item_s1, const int32_t* item_part,
                               int32_t num_part, void* partials, const int32_t* near_off, const int32_t* near_src,
+                              const uint8_t* active,
                               double eps2, double G, void* grad4);
 int32_t jfm_p2p_adjoint_reduce(void* stream, int32_t dtype, const void* cot4, int32_t n, int32_t leaf_size,
                                int32_t num_split, const int32_t* split_leaf, const int32_t* split_p0,
@@ -449,7 +455,8 @@ int32_t jfm_center_adjoint(void* stream, int32_t dtype, int32_t p, const int32_t
  * lane under jax.grad, mutual/force.py:962-1068). */
 int32_t jfm_p2p_adjoint_weighted(void* stream, int32_t dtype, const void* pos4, const void* cot4, int32_t n,
                                  int32_t num_leaves, int32_t leaf_size, const int32_t* near_off,
-                                 const int32_t* near_src, const int32_t* rung_sorted, const void* level_weights,
+                                 const int32_t* near_src,
+                              const uint8_t* active, const int32_t* rung_sorted, const void* level_weights,
                                  int32_t num_levels, double eps2, double G, void* grad4);
 /* jfm_p2p_adjoint_weighted over work items (as jfm_p2p_adjoint_items; the
  * split leaves' partials go through jfm_p2p_adjoint_reduce). */
@@ -457,7 +464,8 @@ int32_t jfm_p2p_adjoint_weighted_items(void* stream, int32_t dtype, const void* 
                                        int32_t num_leaves, int32_t leaf_size, int32_t num_items,
                                        const int32_t* item_leaf, const int32_t* item_s0, const int32_t* item_s1,
                                        const int32_t* item_part, int32_t num_part, void* partials,
-                                       const int32_t* near_off, const int32_t* near_src, const int32_t* rung_sorted,
+                                       const int32_t* near_off, const int32_t* near_src,
+                              const uint8_t* active, const int32_t* rung_sorted,
                                        const void* level_weights, int32_t num_levels, double eps2, double G,
                                        void* grad4);
 int32_t jfm_center_adjoint_weighted(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, int32_t num_nodes,

@@ -28,7 +28,7 @@ MAX_ORDER = 8
 M2L_VALU = 0
 M2L_MFMA = 1
 M2L_ENGINES = {"valu": M2L_VALU, "mfma": M2L_MFMA}
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _i32p = POINTER(c_int32)
 _f64p = POINTER(c_double)
@@ -120,11 +120,12 @@ _SIGNATURES = {
     "jfm_direct_scratch_doubles": (c_int64, [c_int32]),
     "jfm_p2p_adjoint_items": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
-                                        c_double, c_double, c_void_p]),
+                                        c_void_p, c_double, c_double, c_void_p]),
+    "jfm_leaf_nonzero": (c_int32, [c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "jfm_p2p_adjoint_reduce": (c_int32, [c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p,
                                          c_void_p, c_void_p, c_double, c_double, c_void_p]),
     "jfm_p2p_adjoint": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p,
-                                  c_void_p, c_double, c_double, c_void_p]),
+                                  c_void_p, c_void_p, c_double, c_double, c_void_p]),
     "jfm_leaf_adjoint_a": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                      c_void_p, c_void_p, c_double, c_void_p, c_void_p]),
     "jfm_center_adjoint": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
@@ -143,12 +144,12 @@ _SIGNATURES = {
     "jfm_mutual_combine": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
                                      c_void_p]),
     "jfm_p2p_adjoint_weighted": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32,
-                                           c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_double, c_double,
-                                           c_void_p]),
+                                           c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_double,
+                                           c_double, c_void_p]),
     "jfm_p2p_adjoint_weighted_items": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                                  c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
-                                                 c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_double, c_double,
-                                                 c_void_p]),
+                                                 c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_double,
+                                                 c_double, c_void_p]),
     "jfm_center_adjoint_weighted": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p,
                                               c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
                                               c_void_p, c_void_p]),

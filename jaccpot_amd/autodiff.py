@@ -127,20 +127,28 @@ def _recompute(fmm, state, s, code):
     return lown
 
 
-def _p2p_adjoint(state, code, s, cot4, grad4):
+def active_leaves(topo, code, s, cot4) -> torch.Tensor:
+    """Flags of the leaves that hold a cotangent: the adjoint P2P skips pairs of leaves without."""
+    flags = torch.empty(topo.num_leaves, dtype=torch.uint8, device=cot4.device)
+    nat.call("jfm_leaf_nonzero", s, code, cot4.data_ptr(), topo.num_particles, topo.num_leaves, topo.leaf_size,
+             flags.data_ptr())
+    return flags
+
+
+def _p2p_adjoint(state, code, s, cot4, active, grad4):
     """Near-field part of the particle gradient into grad4 (written, not added)."""
     topo = state.topology
     n = topo.num_particles
     items = state.extra.get("p2p_items")
     if items is None:
         nat.call("jfm_p2p_adjoint", s, code, state.pos4.data_ptr(), cot4.data_ptr(), n, topo.num_leaves,
-                 topo.leaf_size, state.near_off.data_ptr(), state.near_src.data_ptr(), state.softening ** 2, state.G,
-                 grad4.data_ptr())
+                 topo.leaf_size, state.near_off.data_ptr(), state.near_src.data_ptr(), active.data_ptr(),
+                 state.softening ** 2, state.G, grad4.data_ptr())
     else:  # long near lists cut into work items, as in the forward P2P
         nat.call("jfm_p2p_adjoint_items", s, code, state.pos4.data_ptr(), cot4.data_ptr(), n, topo.num_leaves,
                  topo.leaf_size, items.num_items, items.leaf.data_ptr(), items.s0.data_ptr(), items.s1.data_ptr(),
                  items.part.data_ptr(), items.num_part, items.partials.data_ptr(), state.near_off.data_ptr(),
-                 state.near_src.data_ptr(), state.softening ** 2, state.G, grad4.data_ptr())
+                 state.near_src.data_ptr(), active.data_ptr(), state.softening ** 2, state.G, grad4.data_ptr())
         nat.call("jfm_p2p_adjoint_reduce", s, code, cot4.data_ptr(), n, topo.leaf_size, items.num_split,
                  items.split_leaf.data_ptr(), items.split_p0.data_ptr(), items.split_p1.data_ptr(),
                  items.partials.data_ptr(), state.softening ** 2, state.G, grad4.data_ptr())
@@ -167,6 +175,7 @@ def fmm_vjp(fmm, state, positions: torch.Tensor, masses: torch.Tensor, acc_bar: 
     pb = pot_bar.to(dev, dt).contiguous()
     nat.call("jfm_gather_sorted", s, code, code, ab.data_ptr(), pb.data_ptr(), state.perm.data_ptr(), n,
              cot4.data_ptr())
+    active = active_leaves(topo, code, s, cot4)
     grad4 = torch.empty((n, 4), dtype=dt, device=dev)
     # the adjoint P2P (most of the work) runs on the overlapped step's P2P
     # stream while this stream recomputes the expansions and runs the tree
@@ -176,7 +185,7 @@ def fmm_vjp(fmm, state, positions: torch.Tensor, masses: torch.Tensor, acc_bar: 
     side = fmm._side_stream(dev)
     side.wait_stream(main)
     with torch.cuda.stream(side):
-        _p2p_adjoint(state, code, nat.current_stream(), cot4, grad4)
+        _p2p_adjoint(state, code, nat.current_stream(), cot4, active, grad4)
     lown = _recompute(fmm, state, s, code)
     grad_l4 = torch.zeros((n, 4), dtype=dt, device=dev)
     lbar = torch.zeros_like(state.locals)

@@ -36,6 +36,7 @@ import numpy as np
 import torch
 
 from . import _native as nat
+from .autodiff import active_leaves
 
 __all__ = [
     "MutualTopology",
@@ -442,7 +443,7 @@ def _near_field(st: MutualFMMState, lw, near: torch.Tensor, code: int, s) -> Non
                  prep.perm.data_ptr(), near.data_ptr())
 
 
-def _near_adjoint(st: MutualFMMState, lw, cot4, grad4, part, code: int, s) -> None:
+def _near_adjoint(st: MutualFMMState, lw, cot4, active, grad4, part, code: int, s) -> None:
     """Near-field part of the particle gradient into grad4 (written, not added);
     ``part``: partials of its own for the work items (None without items)."""
     prep = st.prepared
@@ -452,15 +453,15 @@ def _near_adjoint(st: MutualFMMState, lw, cot4, grad4, part, code: int, s) -> No
     it = st.near_items
     if it is None and lw is not None:
         nat.call("jfm_p2p_adjoint_weighted", s, code, prep.pos4.data_ptr(), cot4.data_ptr(), n, L, ls,
-                 prep.near_off.data_ptr(), prep.near_src.data_ptr(), st.buffers["rung_sorted"].data_ptr(),
-                 lw.data_ptr(), int(lw.numel()), eps2, st.G, grad4.data_ptr())
+                 prep.near_off.data_ptr(), prep.near_src.data_ptr(), active.data_ptr(),
+                 st.buffers["rung_sorted"].data_ptr(), lw.data_ptr(), int(lw.numel()), eps2, st.G, grad4.data_ptr())
     elif it is None:
         nat.call("jfm_p2p_adjoint", s, code, prep.pos4.data_ptr(), cot4.data_ptr(), n, L, ls,
-                 prep.near_off.data_ptr(), prep.near_src.data_ptr(), eps2, st.G, grad4.data_ptr())
+                 prep.near_off.data_ptr(), prep.near_src.data_ptr(), active.data_ptr(), eps2, st.G, grad4.data_ptr())
     else:  # long near lists cut into the forward's work items
         head = (s, code, prep.pos4.data_ptr(), cot4.data_ptr(), n, L, ls, it.num_items, it.leaf.data_ptr(),
                 it.s0.data_ptr(), it.s1.data_ptr(), it.part.data_ptr(), it.num_part, part.data_ptr(),
-                prep.near_off.data_ptr(), prep.near_src.data_ptr())
+                prep.near_off.data_ptr(), prep.near_src.data_ptr(), active.data_ptr())
         if lw is not None:
             nat.call("jfm_p2p_adjoint_weighted_items", *head, st.buffers["rung_sorted"].data_ptr(), lw.data_ptr(),
                      int(lw.numel()), eps2, st.G, grad4.data_ptr())
@@ -490,6 +491,7 @@ def _vjp(st: MutualFMMState, x: torch.Tensor, m: torch.Tensor, lw, acc_bar: torc
     nat.call("jfm_gather_sorted", s, code, code, ab.data_ptr(), pb.data_ptr(), prep.perm.data_ptr(), n,
              cot4.data_ptr())
     grad4 = torch.empty((n, 4), dtype=dt, device=dev)
+    active = active_leaves(topo, code, s, cot4)
     part = torch.empty_like(st.near_items.partials) if st.near_items is not None else None
     # the adjoint near field runs on the P2P stream of the device while this
     # stream recomputes the expansions and runs the tree adjoints; the L2P
@@ -498,9 +500,9 @@ def _vjp(st: MutualFMMState, x: torch.Tensor, m: torch.Tensor, lw, acc_bar: torc
 
     main = torch.cuda.current_stream(dev)
     side = FastMultipoleMethod._side_stream(dev)
-    side.wait_stream(main)
+    side.wait_stream(main)  # after the flags as well
     with torch.cuda.stream(side):
-        _near_adjoint(st, lw, cot4, grad4, part, code, nat.current_stream())
+        _near_adjoint(st, lw, cot4, active, grad4, part, code, nat.current_stream())
     lown = _expansions(st, x, m, lw, gathered=True)
     grad_l4 = torch.zeros((n, 4), dtype=dt, device=dev)
     lbar = torch.zeros_like(prep.locals)
