@@ -222,13 +222,17 @@ def check(rc: int, name: str) -> None:
         raise JfmError(f"{name} failed ({rc}): {msg.decode() if msg else ''}")
 
 
+# entry points that return a value, not a status
+_VALUES = frozenset((
+    "jfm_direct_scratch_doubles", "jfm_coeff_stride", "jfm_order_supported", "jfm_abi_version", "jfm_mlp_num_params",
+    "jfm_mlp_backward_scratch_floats", "jfm_tree_bounds_scratch_doubles", "jfm_key_bits", "jfm_tree_radius_work",
+    "jfm_tree_walk_state_words", "jfm_m2l_engine", "jfm_direct_sum_f64_static_max_targets"))
+
+
 def call(name: str, *args) -> int:
     """Call an entry point and raise JfmError on a non-zero status."""
-    rc = getattr(load(), name)(*args)
-    if name not in ("jfm_direct_scratch_doubles", "jfm_coeff_stride", "jfm_order_supported", "jfm_abi_version",
-                    "jfm_mlp_num_params", "jfm_mlp_backward_scratch_floats", "jfm_tree_bounds_scratch_doubles",
-                    "jfm_key_bits", "jfm_tree_radius_work", "jfm_tree_walk_state_words", "jfm_m2l_engine",
-                    "jfm_direct_sum_f64_static_max_targets"):
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != JFM_OK and name not in _VALUES:
         check(rc, name)
     return rc
 

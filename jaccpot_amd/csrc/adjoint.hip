@@ -154,7 +154,6 @@ constexpr int kMaxLevelWeights = 64;
 // target leaf, the active ones for any other.  A loss over 1024 of 1M bodies
 // (leaf 32) leaves 6% of the pairs: forward and backward 15.0 -> 6.8 ms; dense
 // cotangents 16.9 -> 16.5 ms.
-
 template <typename T, int WT, bool SAFE, bool WEIGHTED = false>
 __global__ __launch_bounds__(kThreads) void p2p_adjoint_kernel(const T* __restrict__ pos4, const T* __restrict__ cot4,
                                                                int32_t n, int32_t leaf_size, uint32_t magic,

@@ -123,6 +123,11 @@ class FastMultipoleMethod:
     # forked onto its own stream (alone, at the full width of the GPU) instead
     # of beside the P2P's workgroups.  Same results either way.
     _p2m_before_near = True
+    # Near-field pairs from which a step runs its P2P on the second stream: the
+    # fork and the join cost the host about 40 us, more than a small P2P lasts
+    # (4096 bodies in float64, 7.3e6 pairs: 118 against 89 us a step; 16k bodies,
+    # 1.1e8 pairs: 67 us of P2P).
+    _fork_pairs = 30_000_000
 
     def __init__(
         self,
@@ -308,6 +313,13 @@ class FastMultipoleMethod:
                                 force_scale_nodes=force_scale_nodes,
                                 runtime_overrides_override=runtime_overrides_override,
                                 fused_device_mode=fused_device_mode, extra=extra)
+        return self._prepare(positions, masses, bounds=bounds, leaf_size=leaf_size, max_order=max_order,
+                             theta=theta)[0]
+
+    def _prepare(self, positions, masses, *, bounds, leaf_size, max_order, theta, expand: bool = True):
+        """(state, None) with the expansions computed, or, for ``expand=False`` and a
+        state built anew at a fixed order, (state, (positions, masses)): the device
+        inputs that a step_device on the state still has to see."""
         p = int(max_order)
         if p < 1 or p > nat.MAX_ORDER:
             raise ValueError(f"max_order must be in [1, {nat.MAX_ORDER}]")
@@ -326,7 +338,7 @@ class FastMultipoleMethod:
                tuple(np.concatenate([np.asarray(bounds[0], float), np.asarray(bounds[1], float)]).tolist()))
         reused = self._try_reuse(key, xd, md, bounds, kind, in_dtype, in_dev)
         if reused is not None:
-            return reused
+            return reused, None
         if self.tree_build == "device":
             topo = build_topology_device(xd, md, leaf_size=int(leaf_size), theta=th, bounds=bounds, check_masses=True)
         else:
@@ -339,7 +351,9 @@ class FastMultipoleMethod:
                                           compensated=self.compensated)
         if self.adaptive_order:
             self._prepare_gears(state, xd, md)
-        self.refresh_prepared_state(state, xd, md)
+        expand = expand or self.adaptive_order
+        if expand:
+            self.refresh_prepared_state(state, xd, md)
         if self.adaptive_order and self.order_judge_targets > 0 and state.extra.get("gears") is not None:
             from .judge import judge_learned_orders
 
@@ -353,7 +367,7 @@ class FastMultipoleMethod:
 
                 codes, _ = sorted_morton(xd, bounds)
             self._reuse = {"key": key, "codes": codes, "state": state, "count": 0}
-        return state
+        return state, None if expand else (xd, md)
 
     def _state_from_topology(self, topo: Topology, p: int, dtype: torch.dtype, th: float, kind: str, in_dtype,
                              in_dev, *, mixed: bool, split_near: bool, G: float, softening: float,
@@ -646,14 +660,17 @@ class FastMultipoleMethod:
         'combine' the join with the P2P stream and the far + near add.
         The zeroing of the locals and the P2M run before the fork, alone on
         the GPU: beside the P2P's workgroups they took 2.5x as long.
-        ``overlap=False`` runs the same launches on the current stream only,
-        P2P after the downward pass, then an accumulating L2P.  In the
+        ``overlap=False``, and a step of few near pairs (``_fork_pairs``), run
+        the same launches on the current stream only, P2P after the downward
+        pass, then an accumulating L2P.  In the
         overlapped order L2P runs before the join into per-state rows
         (unscaled) that jfm_l2p_combine adds to the near-field rows after it,
         with the accumulating L2P's expression (acc += -G * far), so both
         orders, and _evaluate_device (also near first, then far), give the
         same bits for any G."""
         topo = state.topology
+        pairs = (topo.num_near_entries + topo.num_leaves) * topo.leaf_size * topo.leaf_size
+        overlap = overlap and pairs >= self._fork_pairs
         main = torch.cuda.current_stream(state.device)
         s = nat.current_stream()
         code = nat.dtype_code(state.dtype)
@@ -766,10 +783,19 @@ class FastMultipoleMethod:
         """Accelerations (and potentials) in input order (solver.py:1292)."""
         if max_acc_derivative_order != 0:
             raise NotImplementedError("acceleration derivatives need the solidfmm basis, which is not built")
-        n = state.num_particles
-        acc = torch.empty((n, 3), dtype=state.dtype, device=state.device)
-        pot = torch.empty((n,), dtype=state.dtype, device=state.device) if return_potential else None
+        acc, pot = self._rows(state, return_potential)
         self._evaluate_device(state, acc, pot)
+        return self._finish(state, acc, pot, target_indices)
+
+    @staticmethod
+    def _rows(state: FMMPreparedState, return_potential: bool):
+        n = state.num_particles
+        return (torch.empty((n, 3), dtype=state.dtype, device=state.device),
+                torch.empty((n,), dtype=state.dtype, device=state.device) if return_potential else None)
+
+    def _finish(self, state: FMMPreparedState, acc: torch.Tensor, pot: Optional[torch.Tensor], target_indices):
+        """The rows asked for, as the caller gave the inputs."""
+        n = state.num_particles
         if target_indices is not None:
             idx = torch.as_tensor(np.asarray(target_indices) if not isinstance(target_indices, torch.Tensor)
                                   else target_indices, device=state.device).long()
@@ -781,7 +807,7 @@ class FastMultipoleMethod:
             if pot is not None:
                 pot = pot.index_select(0, idx)
         acc = self._to_output(state, acc)
-        if return_potential:
+        if pot is not None:
             return acc, self._to_output(state, pot)
         return acc
 
@@ -855,20 +881,27 @@ class FastMultipoleMethod:
         the reference's: an array mutated in place is not noticed).  The state
         is cached with its key (fmm_derivatives.py:141-185), so direct
         ``prepare_state`` calls in between do not change what is reused."""
+        if max_acc_derivative_order != 0:
+            raise NotImplementedError("acceleration derivatives need the solidfmm basis, which is not built")
         args = (int(leaf_size), int(max_order), theta)
         last = self._last_inputs
+        live = None
         if (reuse_prepared_state and bounds is None and last is not None
                 and last[0]() is positions and last[1]() is masses and last[2] == args):
             state = last[3]
         else:
-            state = self.prepare_state(positions, masses, bounds=bounds, leaf_size=leaf_size, max_order=max_order,
-                                       theta=theta)
-            try:
-                self._last_inputs = (weakref.ref(positions), weakref.ref(masses), args, state)
-            except TypeError:  # objects without weak references (lists) are never reused
-                self._last_inputs = None
-        return self.evaluate_prepared_state(state, target_indices=target_indices, return_potential=return_potential,
-                                            max_acc_derivative_order=max_acc_derivative_order)
+            state, live = self._prepare(positions, masses, bounds=bounds, leaf_size=leaf_size, max_order=max_order,
+                                        theta=theta, expand=False)
+        acc, pot = self._rows(state, return_potential)
+        if live is None:
+            self._evaluate_device(state, acc, pot)
+        else:  # expansions and near field in one step: the P2P runs beside the tree passes
+            self.step_device(state, *live, acc, pot)
+        try:
+            self._last_inputs = (weakref.ref(positions), weakref.ref(masses), args, state)
+        except TypeError:  # objects without weak references (lists) are never reused
+            self._last_inputs = None
+        return self._finish(state, acc, pot, target_indices)
 
 
 class EvaluationGraph:
