@@ -66,8 +66,10 @@ __host__ __device__ __forceinline__ T dev_sqrt(T x) {
 // 1/sqrt(x) for x > 0.  float32: v_rsq_f32 (about 1 ulp); float64: the v_rsq_f64
 // estimate y with one third-order step, y (1 + e/2 + 3e^2/8) with e = 1 - x y^2
 // (the relative error is cubed), 7 instructions against about 35 of a square root
-// and a division.  The minimum turns the NaN of x = inf and x = 0 into e = 1, which
-// leaves y = 0 and y = inf.
+// and a division, and closer to the exact value than these: rms 0.47 against 0.60
+// and at most 1.25 against 1.49 times 2^-53 over 4e6 values in 2^-60..2^20.  The
+// minimum turns the NaN of x = inf and x = 0 into e = 1, which leaves y = 0 and
+// y = inf.
 template <typename T>
 __device__ __forceinline__ T fast_rsqrt(T x) {
   if constexpr (sizeof(T) == 4) {
