@@ -465,14 +465,14 @@ __device__ inline void walk_tile(const Walk& w, const int2* __restrict__ in, int
                                  int2* __restrict__ out, Reserve reserve) {
   constexpr int WAVES = THREADS / 64;
   constexpr int CELLS = MAXR * WAVES;
-  static_assert(CELLS <= 64, "one wave scans the cells");
-  __shared__ int32_t cell[3][64];
+  constexpr int PER = (CELLS + 63) / 64;  // cells of a lane of the wave that scans them
+  __shared__ int32_t cell[3][64 * PER];
   __shared__ int64_t start[3];
   const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
   const uint64_t below = (uint64_t(1) << lane) - 1;
   uint64_t codes = 0;
-  if (tid < 64)
-    for (int c = 0; c < 3; ++c) cell[c][tid] = 0;
+  for (int c = 0; c < 3; ++c)
+    for (int k = tid; k < 64 * PER; k += THREADS) cell[c][k] = 0;
   __syncthreads();
 #pragma unroll 4
   for (int r = 0; r < rounds; ++r) {
@@ -492,13 +492,19 @@ __device__ inline void walk_tile(const Walk& w, const int2* __restrict__ in, int
     int32_t total[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const int32_t own = cell[c][lane];
+      int32_t own = 0;
+      for (int k = 0; k < PER; ++k) own += cell[c][lane * PER + k];
       int32_t v = own;
       for (int o = 1; o < 64; o <<= 1) {
         const int32_t u = __shfl_up(v, o);
         if (lane >= o) v += u;
       }
-      cell[c][lane] = v - own;
+      int32_t at = v - own;
+      for (int k = 0; k < PER; ++k) {
+        const int32_t count = cell[c][lane * PER + k];
+        cell[c][lane * PER + k] = at;
+        at += count;
+      }
       total[c] = __shfl(v, 63);
     }
     if (lane < 3) start[lane] = reserve(lane, lane == 0 ? total[0] : lane == 1 ? total[1] : total[2]);
@@ -538,11 +544,16 @@ __device__ inline void walk_tile(const Walk& w, const int2* __restrict__ in, int
   __syncthreads();  // cell and start are reused by the next tile
 }
 
-// One breadth-first step over a fixed grid.  Tiles grow with the frontier (up
-// to 4096 items), since each adds to the three shared counters once.
-constexpr int kWalkThreads = 256;
+// One breadth-first step over a fixed grid.  Bound by the additions to the three
+// shared counters, one each for a tile and one after another across the XCDs: so
+// one workgroup of 1024 threads per CU, with tiles that grow with the frontier (up
+// to 16384 items), instead of four of 256 (up to 4096 items): 1M Plummer bodies, leaf
+// 16, 48 steps 1400 -> 1136 us; a 256k galaxy, 72 steps 787 -> 560 us; two of 512
+// take 1201 and 606 us.  Loads of four rounds issued together changed nothing at 1M
+// and cost 200 us in the galaxy's short steps.
+constexpr int kWalkThreads = 1024;
 constexpr int kWalkRounds = 16;
-constexpr int kWalkBlocks = 1024;
+constexpr int kWalkBlocks = 256;
 
 __global__ void __launch_bounds__(kWalkThreads) walk_step_kernel(Walk w, int32_t step) {
   unsigned long long* now = w.st + kSteps + 2 * step;

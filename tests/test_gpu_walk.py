@@ -33,6 +33,24 @@ def test_walk_grows_its_buffers(monkeypatch, require_gpu, first, group, n, leaf)
         assert np.array_equal(getattr(dev, f), getattr(host, f)), f
 
 
+@pytest.mark.parametrize("n,leaf,theta", (
+    (1100, 1, 0.7),  # frontiers of a few items a workgroup
+    (160001, 3, 0.7),  # tiles of some rounds, the last one partly filled
+    (700001, 8, 0.6),  # frontiers of more than 256 full tiles
+))
+def test_walk_tiles(require_gpu, n, leaf, theta):
+    from jaccpot_amd import dtopology
+    from jaccpot_amd.topology import build_topology
+
+    x, m = ics.plummer(n, 12)
+    host = build_topology(x, m, leaf_size=leaf, theta=theta)
+    dev = dtopology.build_topology_device(torch.as_tensor(x, device="cuda"), torch.as_tensor(m, device="cuda"),
+                                          leaf_size=leaf, theta=theta)
+    print(f"n {n} leaf {leaf}: {host.num_far_pairs} far, {host.num_near_entries} near", flush=True)
+    for f in ("far_off", "far_src", "near_off", "near_src"):
+        assert np.array_equal(getattr(dev, f), getattr(host, f)), f
+
+
 @pytest.mark.parametrize("n,leaf,chunk", ((3000, 8, 64), (3000, 7, 96), (3000, 8, 8192), (200, 16, 16), (5, 8, 8)))
 def test_device_items_match_host(require_gpu, n, leaf, chunk):
     """Work items cut on the device: every list equal to the host's (None where no leaf is cut)."""
