@@ -560,7 +560,11 @@ __global__ void __launch_bounds__(kWalkThreads) walk_step_kernel(Walk w, int32_t
   const int64_t n = static_cast<int64_t>(now[0]);
   const int buf = static_cast<int>(now[1]);
   if (blockIdx.x == 0 && threadIdx.x == 0) now[3] = n > 0 ? 1 - buf : buf;
-  if (n == 0 || w.st[kOverflow] & kFullFrontier) return;  // unwritten frontier entries are never read
+  // A frontier that did not fit shows in the count that the launch before left (the
+  // unwritten entries are never read; this step leaves 0 items for the next).  The
+  // overflow word would not do: other workgroups of this launch set it meanwhile, and
+  // the waves of one workgroup have to leave together.
+  if (n == 0 || n > w.frontier_cap) return;
   const int64_t most = int64_t(gridDim.x) * kWalkThreads;
   const int rounds = static_cast<int>(min(int64_t(kWalkRounds), (n + most - 1) / most));
   const int64_t tile = int64_t(rounds) * kWalkThreads;
@@ -588,7 +592,7 @@ __global__ void __launch_bounds__(kWalkSmallThreads) walk_small_kernel(Walk w, i
   unsigned long long* now = w.st + kSteps + 2 * step;
   int64_t n = static_cast<int64_t>(now[0]);
   int buf = static_cast<int>(now[1]);
-  bool full = (w.st[kOverflow] & kFullFrontier) != 0;
+  bool full = n > w.frontier_cap;
   if (threadIdx.x == 0) {
     next[1] = static_cast<int64_t>(w.st[kFarCount]);
     next[2] = static_cast<int64_t>(w.st[kNearCount]);

@@ -33,6 +33,23 @@ def test_walk_grows_its_buffers(monkeypatch, require_gpu, first, group, n, leaf)
         assert np.array_equal(getattr(dev, f), getattr(host, f)), f
 
 
+@pytest.mark.parametrize("n,leaf,theta", ((20000, 8, 0.3), (50001, 16, 0.3), (100000, 16, 0.4)))
+def test_walk_at_small_angles(monkeypatch, require_gpu, n, leaf, theta):
+    """Opening angles whose frontier outgrows 96 items a leaf, the first buffer: every
+    workgroup leaves the steps after it as a whole and the walk is repeated."""
+    from jaccpot_amd import dtopology
+    from jaccpot_amd.topology import build_topology
+
+    monkeypatch.setattr(dtopology, "WALK_FIRST", ((448, 128), (960, 320), (96, 32)))
+    x, m = ics.plummer(n, 13)
+    host = build_topology(x, m, leaf_size=leaf, theta=theta)
+    dev = dtopology.build_topology_device(torch.as_tensor(x, device="cuda"), torch.as_tensor(m, device="cuda"),
+                                          leaf_size=leaf, theta=theta)
+    print(f"n {n} leaf {leaf} theta {theta}: {host.num_far_pairs} far, {host.num_near_entries} near", flush=True)
+    for f in ("far_off", "far_src", "near_off", "near_src"):
+        assert np.array_equal(getattr(dev, f), getattr(host, f)), f
+
+
 @pytest.mark.parametrize("n,leaf,theta", (
     (1100, 1, 0.7),  # frontiers of a few items a workgroup
     (160001, 3, 0.7),  # tiles of some rounds, the last one partly filled
