@@ -219,14 +219,19 @@ __global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ 
   T acc[C];
 #pragma unroll
   for (int j = 0; j < C; ++j) acc[j] = T(0);
-  // every lane stays in the loop to the wave's last round (the matrix
-  // instructions, the wave-wide vote and the reduction inside need the whole
-  // wave); lanes past the list repeat the target's first pair and drop the result
+  // The matrix instructions, and the reduction inside the direct form, need every
+  // lane to the wave's last round: lanes past the list repeat the target's first
+  // pair and drop the result.  On the cascade such lanes leave: a drop would hold all
+  // of w beside acc for the select (float32 order 6 / 8: 190 / 280 registers against
+  // 154 / 204, 590 against 340 us for the order-8 pairs of 262k bodies, leaf 16;
+  // float64 order 8 spilled).
+  constexpr bool kLeave = !MF && G > kDirectM2L;
   const int rounds = (e - b + kWave - 1) / kWave;
   bool stored = ACC;  // the row holds sums already (uniform)
   for (int q = 0; q < rounds; ++q) {
     const int k = b + q * kWave + lane;
     const bool live = k < e;
+    if (kLeave && !live) break;
     const int src = far_src[live ? k : b];
     const V4<T> cs4 = load4(centers4, src);
     T v[C];
@@ -252,7 +257,7 @@ __global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ 
     } else {
       T w[C];
       m2l_pair<T, G, MF>(v, w, dx, dy, dz, bu);
-      if (live) {
+      if (kLeave || live) {
 #pragma unroll
         for (int j = 0; j < C; ++j) acc[j] += w[j];
       }
