@@ -174,11 +174,51 @@ __device__ __forceinline__ void m2l_pair(T* v, T* w, T dx, T dy, T dz, const BuR
   }
 }
 
-// Sum of the lanes' coefficients acc[C] added to (ACC) or stored in `row`,
-// through LDS, CH coefficients at a time, lanes in order.
-template <typename T, int C, bool ACC>
-__device__ __forceinline__ void reduce_lanes(const T* acc, T (*red)[row_for(C, sizeof(T))], T* row, int lane) {
+// G <= P is the pair's expansion order (gear): the source multipole is read
+// to degree G, translated at order G and added into degrees <= G of the
+// target local.  ACC adds into the existing rows instead of overwriting them
+// (used when a target's pairs are split across several gears).
+template <typename T, int P, int G, bool ACC, bool MF>
+__global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ targets,
+                                                    const int32_t* __restrict__ far_off,
+                                                    const int32_t* __restrict__ far_src, const T* __restrict__ mult,
+                                                    const T* __restrict__ centers4, T* __restrict__ locals,
+                                                    int32_t cs) {
+  constexpr int C = ncoef(G);
   constexpr int CH = chunk_for(C, sizeof(T));
+  __shared__ T red[kWave][row_for(C, sizeof(T))];
+  const int tgt = targets[xcd_contiguous(blockIdx.x, gridDim.x)];
+  const int lane = threadIdx.x;
+  BuRegs bu;
+  if constexpr (MF) bu.load(lane);
+  const int b = far_off[tgt], e = far_off[tgt + 1];
+  const V4<T> ct = load4(centers4, tgt);
+  T* row = locals + static_cast<int64_t>(tgt) * cs;
+  T acc[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j) acc[j] = T(0);
+  // MF: the matrix instructions need every lane of the wave, so the loop runs
+  // to the wave's last round; lanes past the list repeat the target's first
+  // pair and drop the result.  Elsewhere such lanes leave: a drop would hold all of
+  // w beside acc for the select (float32 order 6 / 8: 190 / 280 registers against
+  // 154 / 204; 590 against 340 us for the order-8 pairs of 262k bodies, leaf 16).
+  const int rounds = (e - b + kWave - 1) / kWave;
+  for (int q = 0; q < rounds; ++q) {
+    const int k = b + q * kWave + lane;
+    if (!MF && k >= e) break;
+    const bool live = k < e;
+    const int src = far_src[live ? k : b];
+    const V4<T> cs4 = load4(centers4, src);
+    T v[C];
+    load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
+    T w[C];
+    m2l_pair<T, G, MF>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
+    if (!MF || live) {
+#pragma unroll
+      for (int j = 0; j < C; ++j) acc[j] += w[j];
+    }
+  }
+  // lane partial sums reduced through LDS, CH coefficients at a time
 #pragma unroll
   for (int c0 = 0; c0 < C; c0 += CH) {
     __syncthreads();
@@ -195,78 +235,6 @@ __device__ __forceinline__ void reduce_lanes(const T* acc, T (*red)[row_for(C, s
         row[c0 + lane] = s;
     }
   }
-}
-
-// G <= P is the pair's expansion order (gear): the source multipole is read
-// to degree G, translated at order G and added into degrees <= G of the
-// target local.  ACC adds into the existing rows instead of overwriting them
-// (used when a target's pairs are split across several gears).
-template <typename T, int P, int G, bool ACC, bool MF>
-__global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ targets,
-                                                    const int32_t* __restrict__ far_off,
-                                                    const int32_t* __restrict__ far_src, const T* __restrict__ mult,
-                                                    const T* __restrict__ centers4, T* __restrict__ locals,
-                                                    int32_t cs) {
-  constexpr int C = ncoef(G);
-  __shared__ T red[kWave][row_for(C, sizeof(T))];
-  const int tgt = targets[xcd_contiguous(blockIdx.x, gridDim.x)];
-  const int lane = threadIdx.x;
-  BuRegs bu;
-  if constexpr (MF) bu.load(lane);
-  const int b = far_off[tgt], e = far_off[tgt + 1];
-  const V4<T> ct = load4(centers4, tgt);
-  T* row = locals + static_cast<int64_t>(tgt) * cs;
-  T acc[C];
-#pragma unroll
-  for (int j = 0; j < C; ++j) acc[j] = T(0);
-  // The matrix instructions, and the reduction inside the direct form, need every
-  // lane to the wave's last round: lanes past the list repeat the target's first
-  // pair and drop the result.  On the cascade such lanes leave: a drop would hold all
-  // of w beside acc for the select (float32 order 6 / 8: 190 / 280 registers against
-  // 154 / 204, 590 against 340 us for the order-8 pairs of 262k bodies, leaf 16;
-  // float64 order 8 spilled).
-  constexpr bool kLeave = !MF && G > kDirectM2L;
-  const int rounds = (e - b + kWave - 1) / kWave;
-  bool stored = ACC;  // the row holds sums already (uniform)
-  for (int q = 0; q < rounds; ++q) {
-    const int k = b + q * kWave + lane;
-    const bool live = k < e;
-    if (kLeave && !live) break;
-    const int src = far_src[live ? k : b];
-    const V4<T> cs4 = load4(centers4, src);
-    T v[C];
-    load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
-    const T dx = ct.x - cs4.x, dy = ct.y - cs4.y, dz = ct.z - cs4.z;  // target - source
-    if constexpr (!MF && G <= kDirectM2L) {
-      // the contributions go straight into the running sums: a dead lane has a
-      // zero multipole, and sums in the way of a rescaled round are stored first
-      if (!live) {
-#pragma unroll
-        for (int j = 0; j < C; ++j) v[j] = T(0);
-      }
-      m2l_direct_add<T, G>(v, acc, dx, dy, dz, [&] {
-        if (q == 0) return;
-        if (stored)
-          reduce_lanes<T, C, true>(acc, red, row, lane);
-        else
-          reduce_lanes<T, C, false>(acc, red, row, lane);
-        stored = true;
-#pragma unroll
-        for (int j = 0; j < C; ++j) acc[j] = T(0);
-      });
-    } else {
-      T w[C];
-      m2l_pair<T, G, MF>(v, w, dx, dy, dz, bu);
-      if (kLeave || live) {
-#pragma unroll
-        for (int j = 0; j < C; ++j) acc[j] += w[j];
-      }
-    }
-  }
-  if (stored)
-    reduce_lanes<T, C, true>(acc, red, row, lane);
-  else
-    reduce_lanes<T, C, false>(acc, red, row, lane);
   if (!ACC)
     for (int j = C + lane; j < cs; j += kWave) row[j] = T(0);
 }

@@ -69,7 +69,8 @@ __host__ __device__ __forceinline__ void irregular_degree(T x, T y, T z, T ir2, 
 }
 
 // Contributions of degree N = n + k of the irregular harmonics (twice them) to
-// w, inputs of degree k <= KMAX; degrees N + 1.. follow by recursion.
+// w, inputs of degree k <= KMAX; degrees N + 1.. follow by recursion.  The monopole's
+// share of degrees 0 and 1, which is most of them, is left to m2l_direct.
 template <typename T, int P, int KMAX, int N>
 __host__ __device__ __forceinline__ void m2l_degrees(const T* v, T* w, T x, T y, T z, T ir2, T start, const T* c1,
                                                      const T* s1, const T* c2, const T* s2) {
@@ -80,14 +81,14 @@ __host__ __device__ __forceinline__ void m2l_degrees(const T* v, T* w, T x, T y,
     // m = 0, l = 0
     const T h = T(0.5) * c[0];
 #pragma unroll
-    for (int k = 0; k <= KTOP; ++k) w[sh_idx(N - k, 0)] = fma(h, v[sh_idx(k, 0)], w[sh_idx(N - k, 0)]);
+    for (int k = N <= 1 ? 1 : 0; k <= KTOP; ++k) w[sh_idx(N - k, 0)] = fma(h, v[sh_idx(k, 0)], w[sh_idx(N - k, 0)]);
     // m > 0, l = 0 and m = 0, l > 0
 #pragma unroll
     for (int m = 1; m <= N; ++m) {
 #pragma unroll
       for (int k = 0; k <= KTOP; ++k) {
         const int n = N - k;
-        if (m <= n) {
+        if (m <= n && !(N == 1 && k == 0)) {
           w[sh_idx(n, m)] = fma(c[m], v[sh_idx(k, 0)], w[sh_idx(n, m)]);
           w[sh_idx(n, -m)] = fma(s[m], v[sh_idx(k, 0)], w[sh_idx(n, -m)]);
         }
@@ -138,13 +139,19 @@ constexpr double pow2(int e) {
   return v;
 }
 
-// w += m2l(v, d) at order P, input degrees above KMAX taken as zero.  Where some
-// active lane's r leaves the safe range, every active lane scales its inputs by
-// r^-k (v is overwritten), takes the harmonics of the unit vector and scales the
-// outputs by r^-(n+1): w must be zero then, so `empty` is called first, which
-// puts w's sum elsewhere and clears it.  Both branches are the same for a wave.
-template <typename T, int P, int KMAX = P, typename Empty>
-__host__ __device__ __forceinline__ void m2l_direct_add(T* v, T* w, T dx, T dy, T dz, Empty empty) {
+// w = m2l(v, d) at order P by the direct form (v is overwritten), input degrees above
+// KMAX taken as zero.  Where some active lane's r leaves the safe range, every active
+// lane scales its inputs by r^-k, takes the harmonics of the unit vector and scales
+// the outputs by r^-(n+1).  Both branches are the same for a wave.
+//
+// Rounding in float32 against 64 bits, direct / cascade, of potential and gradient of
+// 20 pairs summed: 7.0e-8 / 6.7e-8 and 1.45e-7 / 1.65e-7 at order 4, 6.6e-8 / 7.1e-8
+// and 1.5e-7 / 1.6e-7 at 5.  It takes three things: a pair's w apart from the running
+// sums (its (P + 1)^2 products a coefficient added to those one by one: 2.6e-7), the
+// largest terms, the monopole's, added last (first: 1.0e-7 against 5.2e-8 of one pair),
+// and a corrected 1 / r (the estimate alone: gradient 1.8e-7).
+template <typename T, int P, int KMAX = P>
+__host__ __device__ __forceinline__ void m2l_direct(T* v, T* w, T dx, T dy, T dz) {
   constexpr T lo = static_cast<T>(pow2(-safe_exponent(P, sizeof(T), true)));
   constexpr T hi = static_cast<T>(pow2(safe_exponent(P, sizeof(T), false)));
   const T r2 = fma(dx, dx, fma(dy, dy, dz * dz));
@@ -154,8 +161,7 @@ __host__ __device__ __forceinline__ void m2l_direct_add(T* v, T* w, T dx, T dy, 
 #else
   const bool rescale = !safe;
 #endif
-  if (rescale) empty();
-  T rinv = T(0);
+  T rinv = T(0), ir;
   if (rescale) {
     if (r2 > T(0)) {
       const T r = dev_sqrt(r2);
@@ -175,21 +181,28 @@ __host__ __device__ __forceinline__ void m2l_direct_add(T* v, T* w, T dx, T dy, 
       for (int m = -k; m <= k; ++m) v[sh_idx(k, m)] *= f;
       f *= rinv;
     }
-  }
-  T ir, ir2;
-  if (rescale) {
-    ir = ir2 = T(1);
+    ir = T(1);
   } else {
 #if defined(__HIP_DEVICE_COMPILE__)
-    // float32: the hardware reciprocal square root (about 1 ulp); r2 is normal here
-    ir = sizeof(T) == 4 ? T(__builtin_amdgcn_rsqf(static_cast<float>(r2))) : T(1) / dev_sqrt(r2);
-#else
-    ir = T(1) / dev_sqrt(r2);
+    if constexpr (sizeof(T) == 4) {  // the hardware estimate (about 1 ulp; r2 is normal here), one Newton step
+      const T y = __builtin_amdgcn_rsqf(r2);
+      ir = fma(T(0.5) * y, fma(-(r2 * y), y, T(1)), y);
+    } else
 #endif
-    ir2 = ir * ir;
+      ir = T(1) / dev_sqrt(r2);
   }
+#pragma unroll
+  for (int j = 0; j < ncoef(P); ++j) w[j] = T(0);
+  const T ir2 = ir * ir, x = dx * ir2, y = dy * ir2, z = dz * ir2;
   const T zero[1] = {T(0)};
-  m2l_degrees<T, P, KMAX, 0>(v, w, dx * ir2, dy * ir2, dz * ir2, ir2, T(2) * ir, zero, zero, zero, zero);
+  m2l_degrees<T, P, KMAX, 0>(v, w, x, y, z, ir2, T(2) * ir, zero, zero, zero, zero);
+  const T mono = ir * v[0];
+  w[0] += mono;
+  if constexpr (P >= 1) {
+    w[sh_idx(1, 0)] = fma(z, mono, w[sh_idx(1, 0)]);
+    w[sh_idx(1, 1)] = fma(x, T(2) * mono, w[sh_idx(1, 1)]);
+    w[sh_idx(1, -1)] = fma(y, T(2) * mono, w[sh_idx(1, -1)]);
+  }
   if (rescale) {
     T f = rinv;
 #pragma unroll
@@ -208,12 +221,10 @@ __host__ __device__ __forceinline__ void m2l_direct_add(T* v, T* w, T dx, T dy, 
 // P2P of the 4M learned workload, whose waves leave about 96 registers a lane free.
 constexpr int kDirectM2L = 5;
 
-template <typename T, int P, int KMAX = P>
+template <typename T, int P, int KMAX = P, int LINE = kDirectM2L>
 __host__ __device__ __forceinline__ void m2l(T* v, T* w, T dx, T dy, T dz) {
-  if constexpr (P <= kDirectM2L) {
-#pragma unroll
-    for (int j = 0; j < ncoef(P); ++j) w[j] = T(0);
-    m2l_direct_add<T, P, KMAX>(v, w, dx, dy, dz, [] {});
+  if constexpr (P <= LINE) {
+    m2l_direct<T, P, KMAX>(v, w, dx, dy, dz);
   } else {
     Align<T, P> a;
     a.init(dx, dy, dz);

@@ -62,6 +62,66 @@ def test_translations_hold_at_every_separation(p, scale):
                         assert np.abs(g - w).max() <= tol * terms, (op, dtype, n)
 
 
+@pytest.mark.parametrize("p", range(2, 6))
+def test_direct_m2l_rounds_no_worse_than_the_cascade(p):
+    """float32 rounding of one M2L against float64, over cells of eight masses at
+    separations of 2.5 to 8 cell sizes: the potential at the target's centre and, with
+    the gradient there, of the direct form and of the rotation cascade.  400 pairs
+    leave the two root mean squares uncertain by 4% each, so 1.15 for the ratio."""
+    rng = np.random.default_rng(p)
+    err = {"m2l": np.zeros(2), "m2l_cascade": np.zeros(2)}
+    for _ in range(400):
+        u = rng.normal(size=3)
+        d = (u / np.linalg.norm(u) * rng.uniform(2.5, 8)).astype(np.float32)
+        M = H.p2m(rng.uniform(-0.5, 0.5, size=(8, 3)), rng.uniform(0.5, 1.5, 8), p).astype(np.float32)
+        ref = _apply("m2l_cascade", p, nat.JFM_F64, M, d)
+        for op, e in err.items():
+            diff = _apply(op, p, nat.JFM_F32, M, d) - ref
+            e += (diff[0] / ref[0]) ** 2, np.sum(diff[1:4] ** 2) / np.sum(ref[1:4] ** 2)
+    ratio = np.sqrt(err["m2l"] / err["m2l_cascade"])
+    print(p, np.sqrt(err["m2l_cascade"] / 400), ratio)
+    assert np.all(ratio <= 1.15), ratio
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", (2, 4, 5))
+def test_m2l_sums_round_no_worse_than_the_cascades(p):
+    """The same over whole far lists (long ones, flat and by target) on the GPU: the
+    local potentials and gradients of the direct engine and of the matrix-core one,
+    which is the cascade, against float64 locals of the same multipoles."""
+    import torch
+
+    from jaccpot_amd import FastMultipoleMethod
+    from jaccpot_amd.flatlist import build_flat_list, pair_targets
+    from oracle import ics
+
+    x, m = ics.plummer(20000, 8)
+    fmm = FastMultipoleMethod(precision="fp32", theta=0.5)
+    st = fmm.prepare_state(torch.as_tensor(x).cuda(), torch.as_tensor(m).cuda(), leaf_size=16, max_order=p)
+    C, topo, s = (p + 1) ** 2, st.topology, nat.current_stream()
+    wide = [torch.zeros((topo.num_nodes, nat.coeff_stride(p, torch.float64)), dtype=torch.float64, device="cuda")
+            for _ in range(2)]
+    wide[0][:, :C] = st.multipoles[:, :C].double()
+    c64 = st.centers4.double()
+    nat.call("jfm_m2l", s, nat.JFM_F64, p, st.m2l_targets.data_ptr(), topo.num_m2l_targets, st.far_off.data_ptr(),
+             st.far_src.data_ptr(), wide[0].data_ptr(), c64.data_ptr(), wide[1].data_ptr())
+    ref = wide[1][:, :C][st.m2l_targets.long()]
+    flat = build_flat_list(pair_targets(st), st.far_src[:topo.num_far_pairs], p, st.dtype, "cuda")
+    for name, lists in (("target", None), ("flat", flat)):
+        st.extra["flat"] = lists
+        err = {}
+        for engine in ("valu", "mfma"):
+            fmm.m2l_engine = engine
+            st.locals.zero_()
+            fmm._m2l(st, s, nat.JFM_F32)
+            diff = st.locals[:, :C][st.m2l_targets.long()].double() - ref
+            err[engine] = np.array([float(torch.sqrt((diff[:, a:b] ** 2).sum() / (ref[:, a:b] ** 2).sum()))
+                                    for a, b in ((0, 1), (1, 4))])
+        print(f"p {p} {name}: cascade {err['mfma']}, ratio {err['valu'] / err['mfma']}", flush=True)
+        assert np.all(err["valu"] <= 1.15 * err["mfma"]), name
+    nat.call("jfm_set_m2l_engine", nat.M2L_VALU)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("p,leaf,exponent", ((4, 4, -18), (4, 16, -18), (3, 8, -23), (5, 8, -14), (4, 8, 18)))
 def test_m2l_outside_the_plain_range(p, leaf, exponent):
