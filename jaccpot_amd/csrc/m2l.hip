@@ -158,9 +158,21 @@ __device__ __forceinline__ void rotate_all_mf(float* v, const Align<float, P>& a
   }
 }
 
+// Highest order whose pairs take the direct form instead of the cascade.  It has fewer
+// instructions up to order 6, but the registers decide how many waves hide the loads:
+// the cascade runs with one to two waves a SIMD more.  M2L pass in us, direct / cascade:
+//   by target, 262k Plummer bodies, leaf 16: float32 order 4 103 / 109, 5 139 / 149;
+//     float64 order 4 177 / 193, 5 354 / 290
+//   flat, the same list: float32 order 4 104 / 114, 5 157 / 146; float64 order 3
+//     125 / 138, 4 230 / 222, 5 448 / 306
+//   flat with weights, 1M Hernquist bodies, leaf 8: float64 order 4 998 / 1059; 131k
+//     bodies: float64 order 5 297 / 192, float32 order 5 107 / 99
+// Both maps of float32 order 5 take the cascade, so that they round alike.
+constexpr int direct_line(int bytes, bool flat, bool weighted) { return bytes == 8 && flat && !weighted ? 3 : 4; }
+
 // One pair's M2L contribution w at order G (v is overwritten); MF: the rotation
 // cascade with B_U on the matrix cores (float32 only), else translate.hpp's form.
-template <typename T, int G, bool MF>
+template <typename T, int G, bool MF, bool FLAT, bool WEIGHTED = false>
 __device__ __forceinline__ void m2l_pair(T* v, T* w, T dx, T dy, T dz, const BuRegs& bu) {
   if constexpr (MF) {
     static_assert(sizeof(T) == 4, "matrix-core B_U is float32 only");
@@ -170,7 +182,7 @@ __device__ __forceinline__ void m2l_pair(T* v, T* w, T dx, T dy, T dz, const BuR
     zm2l<T, G>(v, w, a.r);
     rotate_all_mf<G, Rot::FromZLocal>(w, a, bu);
   } else {
-    m2l<T, G>(v, w, dx, dy, dz);
+    m2l<T, G, G, direct_line(sizeof(T), FLAT, WEIGHTED)>(v, w, dx, dy, dz);
   }
 }
 
@@ -212,7 +224,7 @@ __global__ __launch_bounds__(kWave) void m2l_kernel(const int32_t* __restrict__ 
     T v[C];
     load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
     T w[C];
-    m2l_pair<T, G, MF>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
+    m2l_pair<T, G, MF, false>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
     if (!MF || live) {
 #pragma unroll
       for (int j = 0; j < C; ++j) acc[j] += w[j];
@@ -289,7 +301,7 @@ __global__ __launch_bounds__(kWave) void m2l_flat_kernel(int32_t K, const int32_
     const V4<T> cs4 = load4(centers4, src);
     T v[C];
     load_row<T, C>(mult + static_cast<int64_t>(src) * cs, v);
-    m2l_pair<T, G, MF>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
+    m2l_pair<T, G, MF, true, WT>(v, w, ct.x - cs4.x, ct.y - cs4.y, ct.z - cs4.z, bu);  // target - source
     if constexpr (WT) {
       const int lv = min(max(max(pw.node_rung[tt], pw.node_rung[src]), 0), pw.nlev - 1);
       const T f = pw.level_w[lv];

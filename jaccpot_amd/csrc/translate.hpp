@@ -214,11 +214,11 @@ __host__ __device__ __forceinline__ void m2l_direct(T* v, T* w, T dx, T dy, T dz
   }
 }
 
-// w = m2l(v, d): the direct form up to order kDirectM2L, the rotation cascade above.
-// Instructions of a float32 pair, direct / cascade: 310 / 500 at order 4, 560 / 720 at
-// 5, 810 / 980 at 6, 1840 / 1740 at 8; registers 73 / 52, 93 / 68, 129 / 88, 263 / 128.
-// At order 6 the flat kernel takes 0.90 ms against 0.53 for the cascade beside the
-// P2P of the 4M learned workload, whose waves leave about 96 registers a lane free.
+// w = m2l(v, d): the direct form up to order LINE, the rotation cascade above.
+// Instructions of a float32 pair, direct / cascade: 340 / 500 at order 4, 600 / 720 at
+// 5, about 850 / 980 at 6 and 1880 / 1740 at 8; registers 73 / 52, 93 / 68, 129 / 88,
+// 263 / 128.  The line is that of the centre adjoints, which translate at the order
+// above the expansions'; the M2L kernels have lines of their own (direct_line).
 constexpr int kDirectM2L = 5;
 
 template <typename T, int P, int KMAX = P, int LINE = kDirectM2L>

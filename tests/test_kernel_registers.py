@@ -46,3 +46,16 @@ def test_m2l_cascade_registers(kernels, t, order, most):
     for name, (vgpr, scratch) in found.items():
         print(name, vgpr, scratch)
         assert vgpr <= most and scratch == 0, name
+
+
+# order 5 where the cascade's waves are worth more than the direct form's instructions:
+# flat at seven waves a SIMD (float32) and four (float64), by target at four and two
+@pytest.mark.parametrize("kernel,t,most", (("m2l_flat_kernel", "f", 72), ("m2l_flat_kernel", "d", 128),
+                                           ("m2l_kernel", "f", 128), ("m2l_kernel", "d", 256)))
+def test_m2l_order_5_registers(kernels, kernel, t, most):
+    valu = "ELb0ELb[01]EEE" if kernel == "m2l_flat_kernel" else "ELb[01]ELb0EEE"  # (engine, weights), (adding, engine)
+    found = {n: v for n, v in kernels.items() if re.search(f"{kernel}I{t}Li5ELi5{valu}", n)}
+    assert len(found) == 2, sorted(found)
+    for name, (vgpr, scratch) in found.items():
+        print(name, vgpr, scratch)
+        assert vgpr <= most and scratch == 0, name
