@@ -643,14 +643,16 @@ int32_t jfm_evaluate(void* stream, int32_t dtype, int32_t p, const void* pos4, i
   if (num_internal != num_leaves - 1) return fail(JFM_ERR_ARG, "jfm_evaluate: num_internal must be L-1");
   if ((flags & JFM_EVAL_POTENTIAL) && !pot) return fail(JFM_ERR_ARG, "jfm_evaluate: pot is NULL");
   void* potp = (flags & JFM_EVAL_POTENTIAL) ? pot : nullptr;
-  if (far) {
-    int32_t rc = jfm_l2p(stream, dtype, p, pos4, n, leaf_size, num_internal, locals, centers4, G, out_index, acc,
-                         potp, 0);
+  // near field first, far field added onto its rows: the order of a step's launches
+  // and of the work items', so that a*G + (-G)*g rounds alike on every path
+  if (near) {
+    int32_t rc = jfm_p2p(stream, dtype, pos4, n, num_leaves, leaf_size, near_off, near_src, eps2, G, out_index, acc,
+                         potp, flags, 0);
     if (rc != JFM_OK) return rc;
   }
-  if (near)
-    return jfm_p2p(stream, dtype, pos4, n, num_leaves, leaf_size, near_off, near_src, eps2, G, out_index, acc, potp,
-                   flags, far ? 1 : 0);
+  if (far)
+    return jfm_l2p(stream, dtype, p, pos4, n, leaf_size, num_internal, locals, centers4, G, out_index, acc, potp,
+                   near ? 1 : 0);
   return JFM_OK;
 }
 
