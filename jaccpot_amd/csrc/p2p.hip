@@ -19,6 +19,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "device_math.hpp"
 #include "launch.hpp"
 #include "rows.hpp"
@@ -28,6 +30,7 @@ namespace jfm {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kWave = 64;
 // LDS per CU is 160 KiB; a workgroup holding just over 1/(N+1) of it caps the
 // CU at N workgroups (LDS is allocated in 512-byte granules).
 constexpr int kLdsPerCu = 160 * 1024;
@@ -293,34 +296,42 @@ __global__ __launch_bounds__(THREADS) void p2p_kernel(const T* __restrict__ pos4
     put_sums<T, POT>(tile[i], xi.w, first, i, leaf_size, part_out, eps2, G, out_index, acc, pot, accumulate, items);
 }
 
+// Waves a SIMD that p2p_any_kernel is compiled for: the kP2PBlocksPerCu workgroups that
+// LDS admits (some instances took 97 to 127 registers, a wave less: float64 leaf 1,
+// uncompensated, 470 us against 355).  One float32 instance has 95 registers either way
+// and a schedule that suits it better without the request (leaf 128: 2.70 against 3.08 ms).
+constexpr int any_waves(int bytes, bool pot, bool comp, bool safe) {
+  return bytes == 4 && !pot && !comp && !safe ? 1 : kP2PBlocksPerCu;
+}
+
 // Any leaf width (1..256), softening and summation.  Thread t owns target
-// t % leaf_size and partition t / leaf_size of floor(256 / leaf_size): with the
+// t % leaf_size and partition t / leaf_size of floor(256 / leaf_size) (at most 64,
+// leaf 1: 32, so that most of the final sums stay in one wave): with the
 // width rounded up to a power of two instead, leaves of 24 left a quarter of the
 // lanes idle.  A tile's first slot is divided by the width once (the same for the
 // workgroup) and the threads' slots by a multiplication with its reciprocal, exact
 // for the at most kThreads + TILE slots of a tile (magic = ceil(2^32 / leaf_size)).
 // Tiles hold tile_slots <= TILE slots, a multiple of 8 rounds of the partitions
 // where they are few, so that full tiles have no remainder of the unrolled loop.
-// 100k bodies, leaf 24, with potentials: 416 -> 318 us.
+// In LDS a partition's slots follow each other (row_len, odd, apart from the next
+// partition's): at a run-time distance every interaction paid an address, 131k Plummer
+// bodies, float32, leaf 24 / 96 / 128 / 256 714 / 3021 / 2825 / 4134 us against
+// 660 / 2758 / 2542 / 3780.
 template <typename T, bool POT, bool COMP, bool SAFE>
-__global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__ pos4, int32_t n, int32_t leaf_size,
-                                                           uint32_t magic, int32_t tile_slots,
-                                                           const int32_t* __restrict__ near_off,
-                                                           const int32_t* __restrict__ near_src, T eps2, T G,
-                                                           const int32_t* __restrict__ out_index,
-                                                           T* __restrict__ acc, T* __restrict__ pot,
-                                                           int32_t accumulate, P2PItems<T> items) {
+__global__ __launch_bounds__(kThreads, any_waves(sizeof(T), POT, COMP, SAFE)) void p2p_any_kernel(
+    const T* __restrict__ pos4, int32_t n, int32_t leaf_size, uint32_t magic, int32_t npart, uint32_t part_magic,
+    int32_t tile_slots, const int32_t* __restrict__ near_off, const int32_t* __restrict__ near_src, T eps2, T G,
+    const int32_t* __restrict__ out_index, T* __restrict__ acc, T* __restrict__ pot, int32_t accumulate,
+    P2PItems<T> items) {
   constexpr int TILE = sizeof(T) == 4 ? 1024 : 512;
   constexpr int LOADS = TILE / kThreads;
-  // past the tile's slots: massless rows for the last round of every partition
-  constexpr int kElems = TILE + kThreads;
+  constexpr int kElems = TILE + kWave;  // at most kWave rows, padded by a slot each
   constexpr int kPadElems = static_cast<int>(kP2PLdsBytes / sizeof(V4<T>));
   __shared__ V4<T> tile[kElems > kPadElems ? kElems : kPadElems];
   const int tid = threadIdx.x;
   const int item = xcd_contiguous(blockIdx.x, gridDim.x);
   const int leaf = items.leaf ? items.leaf[item] : item;
   auto quotient = [&](uint32_t v) { return leaf_size == 1 ? v : __umulhi(v, magic); };
-  const int npart = kThreads / leaf_size;
   int part = static_cast<int>(quotient(tid));
   const int i = tid - part * leaf_size;
   const bool idle = part >= npart;
@@ -364,7 +375,14 @@ __global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__
   fetch_list(start);
   fetch_positions(start);
   fetch_list(start + tile_slots);
-  tile[TILE + tid] = V4<T>{T(0), T(0), T(0), T(0)};
+  const int row_len = static_cast<int>(npart == 1 ? tile_slots : __umulhi(tile_slots, part_magic)) | 1;
+  int at[LOADS];  // where this thread's slots of a tile lie (-1: past its slots)
+#pragma unroll
+  for (int l = 0; l < LOADS; ++l) {
+    const int v = tid + l * kThreads;
+    const int k = npart == 1 ? v : static_cast<int>(__umulhi(v, part_magic));
+    at[l] = v < tile_slots ? (v - k * npart) * row_len + k : -1;
+  }
 
   T sx = 0, sy = 0, sz = 0, sp = 0;
   T kx = 0, ky = 0, kz = 0, kp = 0;
@@ -374,7 +392,7 @@ __global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__
     for (int l = 0; l < LOADS; ++l) {
       V4<T> q = next[l];
       if (!ok[l]) q.w = T(0);
-      tile[l * kThreads + tid] = q;
+      if (at[l] >= 0) tile[at[l]] = q;
     }
     __syncthreads();
     // unconditional, as in p2p_kernel: past the end they yield massless slots
@@ -382,10 +400,10 @@ __global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__
     fetch_list(base + 2 * tile_slots);
     const int trips = (min(tile_slots, total - base) + npart - 1) / npart;
     T tx = 0, ty = 0, tz = 0, tp = 0;
-    const V4<T>* src = tile + part;
+    const V4<T>* src = tile + part * row_len;
 #pragma unroll 8
-    for (int k = 0; k < trips; ++k, src += npart) {
-      const V4<T> s = *src;
+    for (int k = 0; k < trips; ++k) {
+      const V4<T> s = src[k];
       const T dx = s.x - xi.x;
       const T dy = s.y - xi.y;
       const T dz = s.z - xi.z;
@@ -416,14 +434,23 @@ __global__ __launch_bounds__(kThreads) void p2p_any_kernel(const T* __restrict__
   __syncthreads();
   int w = 1;
   while (2 * w < npart) w *= 2;  // pairwise over the partitions, fixed order
-  for (; w >= 1; w >>= 1) {
+  auto fold = [&] {
     if (!idle && part < w && part + w < npart) {
       const V4<T> a = tile[tid];
       const V4<T> b = tile[tid + w * leaf_size];
       tile[tid] = V4<T>{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
     }
+  };
+  for (; w * leaf_size > kWave; w >>= 1) {
+    fold();
     __syncthreads();
   }
+  if (tid < kWave)  // the rest within the first wave, whose LDS operations stay in order
+    for (; w >= 1; w >>= 1) {
+      fold();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   if (!idle && part == 0 && i < cnt)
     put_sums<T, POT>(tile[i], xi.w, first, i, leaf_size, part_out, eps2, G, out_index, acc, pot, accumulate, items);
 }
@@ -500,16 +527,16 @@ void launch_p2p_any(hipStream_t s, const T* pos4, int32_t n, int32_t leaf_size, 
                     const int32_t* near_off, const int32_t* near_src, T eps2, T G, const int32_t* out_index, T* acc,
                     T* pot, bool comp, bool accumulate, P2PItems<T> items) {
   const bool safe = !(eps2 > T(0));
-  const uint32_t magic = static_cast<uint32_t>(((uint64_t(1) << 32) + leaf_size - 1) / leaf_size);
+  auto reciprocal = [](int d) { return static_cast<uint32_t>(((uint64_t(1) << 32) + d - 1) / d); };
+  const uint32_t magic = reciprocal(leaf_size);
   constexpr int kTile = sizeof(T) == 4 ? 1024 : 512;
-  const int npart = kThreads / leaf_size;
+  const int npart = leaf_size == 1 ? 32 : std::min(kThreads / leaf_size, kWave);
   const int round = npart <= 32 ? 8 * npart : 4 * npart <= kTile ? 4 * npart : npart;
   const int tile_slots = kTile - kTile % round;
-#define JFM_P2P_ANY(COMP, SAFE)                                                                              \
-  p2p_any_kernel<T, POT, COMP, SAFE><<<num_blocks, kThreads, 0, s>>>(pos4, n, leaf_size, magic, tile_slots, \
-                                                                     near_off, near_src, eps2, G,          \
-                                                                     out_index, acc, pot,                  \
-                                                                     accumulate ? 1 : 0, items)
+#define JFM_P2P_ANY(COMP, SAFE)                                                                                   \
+  p2p_any_kernel<T, POT, COMP, SAFE><<<num_blocks, kThreads, 0, s>>>(                                             \
+      pos4, n, leaf_size, magic, npart, reciprocal(npart), tile_slots, near_off, near_src, eps2, G, out_index, acc, \
+      pot, accumulate ? 1 : 0, items)
   if (comp && safe)
     JFM_P2P_ANY(true, true);
   else if (comp)

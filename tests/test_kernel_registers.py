@@ -1,4 +1,4 @@
-"""Registers of the M2L kernels in the built library (their code objects' metadata):
+"""Registers of M2L and P2P kernels in the built library (their code objects' metadata):
 a SIMD holds 512 vector registers a lane, so a kernel's count decides its waves."""
 
 from __future__ import annotations
@@ -59,3 +59,11 @@ def test_m2l_order_5_registers(kernels, kernel, t, most):
     for name, (vgpr, scratch) in found.items():
         print(name, vgpr, scratch)
         assert vgpr <= most and scratch == 0, name
+
+
+def test_p2p_any_registers(kernels):
+    """Every instance runs the five waves a SIMD that its LDS admits."""
+    found = {n: v for n, v in kernels.items() if "p2p_any_kernel" in n}
+    assert len(found) == 16
+    for name, (vgpr, scratch) in found.items():
+        assert vgpr <= 96 and scratch == 0, (name, vgpr, scratch)
