@@ -275,9 +275,9 @@ class FastMultipoleMethod:
         else:
             x_np = np.asarray(positions)
             kind, in_dtype, in_dev = "numpy", x_np.dtype, None
-            # float32 arrays are widened on the GPU
-            x = torch.as_tensor(np.asarray(x_np, x_np.dtype if x_np.dtype == np.float32 else np.float64))
-            m = torch.as_tensor(np.asarray(masses, np.float64))
+            # float32 arrays are widened on the GPU; torch wants writable arrays without negative strides
+            x = torch.as_tensor(np.require(x_np, np.float32 if x_np.dtype == np.float32 else np.float64, "CW"))
+            m = torch.as_tensor(np.require(masses, np.float64, "CW"))
         if x.ndim != 2 or x.shape[1] != 3:
             raise ValueError("positions must have shape (N, 3)")
         if m.shape != (x.shape[0],):
