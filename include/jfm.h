@@ -256,8 +256,9 @@ int32_t jfm_m2m_level(void* stream, int32_t dtype, int32_t p, const int32_t* nod
 /* Every level of the upward pass, in order: level l holds nodes
  * [lev_off_host[l], lev_off_host[l + 1]) of the level-ordered list `nodes`
  * (deepest first; lev_off_host is host memory, read before the call returns).
- * The same rows as one jfm_m2m_level per level; runs of small levels share a
- * launch. */
+ * Runs of small levels share a launch.  The rows of one jfm_m2m_level per level,
+ * at orders 6 to 8 to rounding: there a narrow level of a run is translated
+ * directly, a level's own launch by rotations. */
 int32_t jfm_m2m_pass(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, const int32_t* lev_off_host,
                      int32_t nlev, const int32_t* left, const int32_t* right, const int32_t* node_range,
                      void* multipoles, void* centers4);
@@ -434,8 +435,7 @@ int32_t jfm_p2p_adjoint_items(void* stream, int32_t dtype, const void* pos4, con
                               int32_t num_leaves, int32_t leaf_size, int32_t num_items, const int32_t* item_leaf,
                               const int32_t* item_s0, const int32_t* item_s1, const int32_t* item_part,
                               int32_t num_part, void* partials, const int32_t* near_off, const int32_t* near_src,
-                              const uint8_t* active,
-                              double eps2, double G, void* grad4);
+                              const uint8_t* active, double eps2, double G, void* grad4);
 int32_t jfm_p2p_adjoint_reduce(void* stream, int32_t dtype, const void* cot4, int32_t n, int32_t leaf_size,
                                int32_t num_split, const int32_t* split_leaf, const int32_t* split_p0,
                                const int32_t* split_p1, const void* partials, double eps2, double G, void* grad4);
@@ -455,19 +455,17 @@ int32_t jfm_center_adjoint(void* stream, int32_t dtype, int32_t p, const int32_t
  * lane under jax.grad, mutual/force.py:962-1068). */
 int32_t jfm_p2p_adjoint_weighted(void* stream, int32_t dtype, const void* pos4, const void* cot4, int32_t n,
                                  int32_t num_leaves, int32_t leaf_size, const int32_t* near_off,
-                                 const int32_t* near_src,
-                              const uint8_t* active, const int32_t* rung_sorted, const void* level_weights,
-                                 int32_t num_levels, double eps2, double G, void* grad4);
+                                 const int32_t* near_src, const uint8_t* active, const int32_t* rung_sorted,
+                                 const void* level_weights, int32_t num_levels, double eps2, double G, void* grad4);
 /* jfm_p2p_adjoint_weighted over work items (as jfm_p2p_adjoint_items; the
  * split leaves' partials go through jfm_p2p_adjoint_reduce). */
 int32_t jfm_p2p_adjoint_weighted_items(void* stream, int32_t dtype, const void* pos4, const void* cot4, int32_t n,
                                        int32_t num_leaves, int32_t leaf_size, int32_t num_items,
                                        const int32_t* item_leaf, const int32_t* item_s0, const int32_t* item_s1,
                                        const int32_t* item_part, int32_t num_part, void* partials,
-                                       const int32_t* near_off, const int32_t* near_src,
-                              const uint8_t* active, const int32_t* rung_sorted,
-                                       const void* level_weights, int32_t num_levels, double eps2, double G,
-                                       void* grad4);
+                                       const int32_t* near_off, const int32_t* near_src, const uint8_t* active,
+                                       const int32_t* rung_sorted, const void* level_weights, int32_t num_levels,
+                                       double eps2, double G, void* grad4);
 int32_t jfm_center_adjoint_weighted(void* stream, int32_t dtype, int32_t p, const int32_t* nodes, int32_t num_nodes,
                                     const int32_t* far_off, const int32_t* far_src, const int32_t* node_rung,
                                     const void* level_weights, int32_t num_levels, const void* multipoles,

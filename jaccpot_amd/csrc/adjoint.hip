@@ -690,8 +690,7 @@ int32_t jfm_p2p_adjoint_items(void* stream, int32_t dtype, const void* pos4, con
                               int32_t num_leaves, int32_t leaf_size, int32_t num_items, const int32_t* item_leaf,
                               const int32_t* item_s0, const int32_t* item_s1, const int32_t* item_part,
                               int32_t num_part, void* partials, const int32_t* near_off, const int32_t* near_src,
-                              const uint8_t* active,
-                              double eps2, double G, void* grad4) {
+                              const uint8_t* active, double eps2, double G, void* grad4) {
   if (n < 1 || leaf_size < 1 || leaf_size > 256 || num_leaves != (n + leaf_size - 1) / leaf_size || num_items < 1 ||
       num_part < 0)
     return fail(JFM_ERR_ARG, "jfm_p2p_adjoint_items: inconsistent sizes");
@@ -791,9 +790,8 @@ int32_t jfm_center_adjoint_weighted(void* stream, int32_t dtype, int32_t p, cons
 
 int32_t jfm_p2p_adjoint_weighted(void* stream, int32_t dtype, const void* pos4, const void* cot4, int32_t n,
                                  int32_t num_leaves, int32_t leaf_size, const int32_t* near_off,
-                                 const int32_t* near_src,
-                              const uint8_t* active, const int32_t* rung_sorted, const void* level_weights,
-                                 int32_t num_levels, double eps2, double G, void* grad4) {
+                                 const int32_t* near_src, const uint8_t* active, const int32_t* rung_sorted,
+                                 const void* level_weights, int32_t num_levels, double eps2, double G, void* grad4) {
   if (n < 1 || leaf_size < 1 || leaf_size > 256 || num_leaves != (n + leaf_size - 1) / leaf_size)
     return fail(JFM_ERR_ARG, "jfm_p2p_adjoint_weighted: inconsistent sizes");
   if (num_levels < 1 || num_levels > kMaxLevelWeights)
