@@ -123,10 +123,11 @@ class FastMultipoleMethod:
     # forked onto its own stream (alone, at the full width of the GPU) instead
     # of beside the P2P's workgroups.  Same results either way.
     _p2m_before_near = True
-    # Near-field pairs from which a step runs its P2P on the second stream: the
-    # fork and the join cost the host about 40 us, more than a small P2P lasts
-    # (4096 bodies in float64, 7.3e6 pairs: 118 against 89 us a step; 16k bodies,
-    # 1.1e8 pairs: 67 us of P2P).
+    # Near-field pairs (a float64 one counts 2.5: it takes as much longer) from
+    # which a step runs its P2P on the second stream.  The fork and the join cost
+    # the host about 40 us, more than a small P2P lasts; us a step, forked / not:
+    # float32 1.4e7 pairs 117 / 84, 2.1e7 117 / 116, 6.1e7 114 / 113, 1.1e8 123 / 141;
+    # float64 8.6e6 118 / 118, 1.4e7 114 / 119, 2.1e7 150 / 172, 6.1e7 144 / 198.
     _fork_pairs = 30_000_000
 
     def __init__(
@@ -669,8 +670,7 @@ class FastMultipoleMethod:
         orders, and _evaluate_device (also near first, then far), give the
         same bits for any G."""
         topo = state.topology
-        pairs = (topo.num_near_entries + topo.num_leaves) * topo.leaf_size * topo.leaf_size
-        overlap = overlap and pairs >= self._fork_pairs
+        overlap = overlap and self._forks(topo, state.dtype)
         main = torch.cuda.current_stream(state.device)
         s = nat.current_stream()
         code = nat.dtype_code(state.dtype)
@@ -734,6 +734,11 @@ class FastMultipoleMethod:
             mark("l2p", 1)
             mark("combine", 0)
             mark("combine", 1)
+
+    def _forks(self, topo: Topology, dtype: torch.dtype) -> bool:
+        """Whether a step's near field is long enough for a stream of its own."""
+        pairs = (topo.num_near_entries + topo.num_leaves) * topo.leaf_size * topo.leaf_size
+        return pairs * (2.5 if dtype == torch.float64 else 1) >= self._fork_pairs
 
     @staticmethod
     def _far_rows(state: FMMPreparedState):
