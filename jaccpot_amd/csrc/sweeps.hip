@@ -376,10 +376,11 @@ __device__ __forceinline__ void for_wave_part(F f) {
 }
 static_assert(kSpanThreads == 4 * kWave, "one wave for each part");
 
-// Whether a level of `count` nodes (`lanes` lanes each) runs in parts.
+// Whether a level of `count` nodes (`lanes` lanes each) runs in parts: a wave's lanes
+// going up, 48 going down (order 7, float32: 64 nodes 6.2 us in parts, 4.5 whole).
 template <int P>
 __device__ __forceinline__ bool by_parts(int count, int lanes) {
-  return P >= kPartOrder && count * lanes <= kWave;
+  return P >= kPartOrder && count * lanes <= (lanes == 2 ? kWave : 48);
 }
 
 template <typename T, int P>
@@ -453,9 +454,22 @@ __global__ __launch_bounds__(kSpanThreads) void l2l_span_kernel(const int32_t* _
   }
 }
 
-// Levels of at most this many nodes join a span: SPAN_ROUNDS passes of the
-// workgroup over a level, which then costs about as much as a launch.
-constexpr int span_rounds(int p) { return p <= 4 ? 2 : 1; }
+// Levels of at most this many nodes join a span.  The lines lie where a level of a span
+// takes as long as one more launch (16 levels of equal width in a pass, us a level, span /
+// launch; the span costs a round trip and rises with each 128 nodes up, 256 down):
+//   up    float32 order 4, 256 nodes: 3.6 / 3.4   order 8, 128: 6.3 / 6.7
+//         float64 order 4, 128: 2.5 / 3.5, 256: 4.7 / 3.6   order 8, 64: 8.1 / 8.3, 128: 9.7 / 8.3
+//   down  float32 order 4, 256: 2.2 / 3.3, 512: 4.3 / 3.3   6, 192: 4.5 / 4.6   8, 128: 6.4 / 6.5
+//         float64 order 4, 192: 3.1 / 3.3, 512: 7.9 / 3.5   6, 128: 5.5 / 5.5   8, 64: 7.5 / 8.0
+// At 32 nodes: 1.5 / 3.3 (order 4) to 3.9 / 6.1 (order 8), float32.
+constexpr int span_nodes_up(int p, int bytes) {
+  if (bytes == 4) return p <= 4 ? 256 : 128;
+  return p <= 3 ? 256 : p <= 6 ? 128 : 64;
+}
+constexpr int span_nodes_down(int p, int bytes) {
+  if (bytes == 4) return p <= 3 ? 512 : p <= 5 ? 256 : p == 6 ? 192 : 128;
+  return p <= 2 ? 512 : p == 3 ? 256 : p <= 5 ? 192 : p == 6 ? 128 : 64;
+}
 
 // One thread per node of a level: L += l2l(L_parent, c_parent - c).
 template <typename T, int P>
@@ -768,7 +782,7 @@ int32_t jfm_m2m_pass(void* stream, int32_t dtype, int32_t p, const int32_t* node
   JFM_FOR_DTYPE(dtype, JFM_FOR_ORDER(p, {
     const int cs = coef_stride(P, sizeof(T));
     for_level_spans(
-        lev_off_host, nlev, span_rounds(P) * kSpanThreads / 2,
+        lev_off_host, nlev, span_nodes_up(P, sizeof(T)),
         [&](const LevelSpan& sp) {
           m2m_span_kernel<T, P><<<1, kSpanThreads, 0, s>>>(nodes, sp, left, right, node_range, (T*)multipoles, cs,
                                                            (T*)centers4);
@@ -790,7 +804,7 @@ int32_t jfm_l2l_pass(void* stream, int32_t dtype, int32_t p, const int32_t* node
   JFM_FOR_DTYPE(dtype, JFM_FOR_ORDER(p, {
     const int cs = coef_stride(P, sizeof(T));
     for_level_spans(
-        lev_off_host, nlev, span_rounds(P) * kSpanThreads,
+        lev_off_host, nlev, span_nodes_down(P, sizeof(T)),
         [&](const LevelSpan& sp) {
           l2l_span_kernel<T, P><<<1, kSpanThreads, 0, s>>>(nodes, sp, parent, (const T*)centers4, (T*)locals, cs);
         },

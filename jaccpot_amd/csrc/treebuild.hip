@@ -291,7 +291,9 @@ __global__ void __launch_bounds__(256) internal_geometry_kernel(Particles P, int
   if (q < count) internal_geometry(P, level_nodes[q], left, right, range, mass, center);
 }
 
-// A run of small levels in one workgroup, a barrier between the levels.
+// A run of small levels in one workgroup, a barrier between the levels.  The line lies
+// where a level takes about as long as one more launch (256 nodes 1.7 us in a run,
+// 1024 3.7; wider ones by themselves 3.5).
 constexpr int kGeometrySpanThreads = 512;
 constexpr int kGeometrySpanNodes = 2 * kGeometrySpanThreads;
 

@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 # each in a run of its own kind: wide, run, wide, run to the end
-WIDTHS = ([300, 33, 32, 1, 2, 65, 64, 129, 128, 257], [513, 600], [256, 31, 5, 127])
+WIDTHS = ([300, 33, 32, 1, 2, 65, 64, 129, 128, 257], [513, 600], [256, 31, 5, 127], [192, 48, 193, 49, 512, 47])
 
 
 def _levels(rng, widths, leaves):
