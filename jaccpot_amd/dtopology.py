@@ -109,7 +109,11 @@ def _key_bits(max_key: int) -> int:
 WALK_GROUP = 12
 # First buffer sizes per leaf (far entries, near entries, frontier items): the
 # longest lists seen on clustered inputs at opening angles from 0.55 are 410, 885
-# and 83.  Where they would pass WALK_LIMIT_BYTES, that or the second figures.
+# and 83.  Where they would pass WALK_LIMIT_BYTES, that or the second figures (4.9
+# GB in all at 524,288 leaves).  Smaller angles find them too small and walk two or
+# three times; a whole build of Plummer bodies takes 0.97 / 1.05 / 1.8 / 1.9 ms at
+# angles 0.6 / 0.5 / 0.4 / 0.3 (65,536 bodies, leaf 16) and 2.1 / 4.1 / 6.7 / 11.7
+# (524,288), where lists grown between the steps took 4.3 to 4.8 and 6.8 to 19.5.
 WALK_FIRST = ((448, 128), (960, 320), (96, 32))
 WALK_LIMIT_BYTES = 1 << 31
 
@@ -125,6 +129,9 @@ def _walk(I: int, nodes: int, L: int, node4: torch.Tensor, left: torch.Tensor, r
     far_cap, near_cap, fcap = (max(1024, min(per * L, max(WALK_LIMIT_BYTES // b, least * L)))
                                for (per, least), b in zip(WALK_FIRST, width + (16,)))
     caps = [far_cap, near_cap]
+    # more groups in the first call spare looks at deep trees and cost shallow ones empty
+    # steps: a build with 1 / 2 / 4 groups takes 642 / 664 / 716 us at 256 leaves, 919 /
+    # 881 / 872 at 1024, 1338 / 1309 / 1208 at 8192, 1641 / 1605 / 1532 at 16,384
     groups = 1 if L <= 1024 else 2 if L <= 8192 else 4
     while True:
         frontier = torch.empty((2, fcap, 2), dtype=torch.int32, device=dev)
