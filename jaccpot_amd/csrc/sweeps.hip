@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kWave) void m2m_kernel(const int32_t* __restrict__ 
 // threads, one wave per SIMD, so that the workgroup finds room on a CU beside the
 // P2P's workgroups (wider ones wait for several of those to end).
 //
-// From order 6 a level of at most a wave's nodes is cut four ways: each wave
+// From order 6 a level of at most 32 nodes (up) or 48 (down) is cut four ways: each wave
 // computes a quarter of every node's outputs (shift_part) by the direct form, 445
 // instructions instead of 1080.  Such a level takes 1.8 us instead of 3.1 at order
 // 6, 3.0 instead of 5.2 at order 8 (float32, upward, 16 nodes; without arithmetic
